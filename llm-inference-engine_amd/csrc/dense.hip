@@ -16,15 +16,17 @@
 // at most 16, then 8, significant bits), and each block is multiplied three
 // times, so every product is the f32-exact w * x. Only the summation order
 // differs from the CPU's: the results agree to float32 rounding of the sum.
-// The 8 waves of a workgroup take interleaved 32-wide K blocks and their
-// partial tiles are added through LDS in a fixed order, so results do not
-// depend on scheduling. Larger launches take several tiles per workgroup
-// (see launch_matmul).
+// matmul_tiled_kernel (matmul_tiled.hpp) is that product with its operands staged in LDS,
+// in one of several tile shapes (see choose_tile), for K in whole 32-wide blocks and
+// weights aligned for the DMA; matmul_mfma_kernel here loads its operands directly, for
+// every other shape. Both add every output in the same order, fixed by the matrix alone.
 // Lane (g, r) of a tile: A = W[row r][k + 8g .. +8], B = x[token r][k + 8g ..
 // +8]; the result lane holds rows 4g .. 4g+3 of token r.
 #include <algorithm>
+#include <iterator>
 
 #include "common.hpp"
+#include "matmul_tiled.hpp"
 #include "mfma.hpp"
 
 namespace iehip {
@@ -32,39 +34,15 @@ namespace {
 
 constexpr int kMmWaves = 8;  // waves of a workgroup, splitting K
 
-using bf16 = __bf16;
-
 template <bool I8>
 __device__ __forceinline__ bf16x8 load_weights(const void* w, size_t idx) {
   bf16x8 a;
   if constexpr (!I8) {
     a = *reinterpret_cast<const bf16x8*>(static_cast<const uint16_t*>(w) + idx);
   } else {
-    const uint2 raw = *reinterpret_cast<const uint2*>(static_cast<const int8_t*>(w) + idx);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const uint32_t word = j < 4 ? raw.x : raw.y;
-      const int8_t q = static_cast<int8_t>((word >> (8 * (j & 3))) & 0xFF);
-      a[j] = static_cast<bf16>(static_cast<float>(q));
-    }
+    a = widen_i8(*reinterpret_cast<const uint2*>(static_cast<const int8_t*>(w) + idx));
   }
   return a;
-}
-
-// 8 activations as three bf16 operands whose sum is exact.
-__device__ __forceinline__ void split3(const float4 p, const float4 q, bf16x8& hi, bf16x8& mid,
-                                       bf16x8& lo) {
-  const float v[8] = {p.x, p.y, p.z, p.w, q.x, q.y, q.z, q.w};
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const bf16 h = static_cast<bf16>(v[j]);
-    const float r1 = v[j] - static_cast<float>(h);
-    const bf16 m = static_cast<bf16>(r1);
-    const float r2 = r1 - static_cast<float>(m);
-    hi[j] = h;
-    mid[j] = m;
-    lo[j] = static_cast<bf16>(r2);
-  }
 }
 
 __device__ __forceinline__ f32x4 mma3(bf16x8 a, bf16x8 bh, bf16x8 bm, bf16x8 bl, f32x4 c) {
@@ -73,43 +51,15 @@ __device__ __forceinline__ f32x4 mma3(bf16x8 a, bf16x8 bh, bf16x8 bm, bf16x8 bl,
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bl, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ float silu(float v) { return v / (1.0f + expf(-v)); }
-
 // GATE: out = silu(x . Wg^T * sg) * (x . Wu^T * su) (gate_up_silu); otherwise
 // y (+)= x . W^T * s + bias. A workgroup owns RT x TT tiles of 16 rows x 16
 // tokens: each weight fragment is loaded once per K block and used for all TT
 // token tiles (so the weights are read once per launch when T <= 16 TT), each
 // activation fragment split once and used for all RT row tiles. cols % 8 == 0;
-// the K tail past cols is zero.
-// Outputs: rows [0, split0) go to y ([T, split0]), rows [split0, split1) to y1
-// ([T, split1 - split0]) and the rest to y2 ([T, rows - split1]); a plain
-// matmul has split0 = split1 = rows.
-struct RowSplit {
-  float* y1;
-  float* y2;
-  int split0, split1;
-};
-
-// NORM: the rmsnorm before the matmul, folded into it (the decode step's
-// xn = rmsnorm(x); y = xn . W^T pairs). y = (x * w_norm) . W^T * inv_rms(x):
-// the activations are scaled by the norm weight as they are split, each lane
-// sums the squares of the raw x it loads, the waves add those sums through LDS
-// in the same fixed tree as their tiles, and the epilogue takes the row's
-// 1 / sqrt(mean(x^2) + eps). The orders depend on the matrix shape alone.
-struct RowNorm {
-  const float* weight;  // [cols]
-  float eps;
-};
-
-// STAGED (the 8-wave, one-token-tile launches; cols % 32 == 0): the K blocks'
-// weight and activation tiles reach each wave's own LDS stages by DMA
-// (global_load_lds_dwordx4) in whole 64-byte row pieces, one block ahead, and
-// the MFMA operands are read back from there. A lane's direct loads of its
-// operands (row r, columns 8g..8g+7) put 16 rows into each quarter-wave, one
-// L1 access per lane; the L1 access rate then bounded these launches (probe,
-// down 896 x 4,864 at 64 tokens: 15.3 us direct, 8.5 us staged). The MFMA
-// operands and their order are the same, so the results are the same bits.
-template <bool GATE, int RT, int TT, int W, bool I8, bool NORM = false, bool STAGED = false>
+// the K tail past cols is zero. Lane (g, r)'s direct loads of its operands touch 16
+// rows per quarter-wave, and the L1's access rate bounds the kernel: shapes that the
+// LDS tiles take run there (down 896 x 4,864 at 64 tokens: 15.3 us here, 8.7 us there).
+template <bool GATE, int RT, int TT, int W, bool I8, bool NORM = false>
 __global__ void __launch_bounds__(64 * W)
 matmul_mfma_kernel(float* __restrict__ y, const float* __restrict__ x, const void* __restrict__ w,
                    const float* __restrict__ scale, const void* __restrict__ w2,
@@ -139,117 +89,6 @@ matmul_mfma_kernel(float* __restrict__ y, const float* __restrict__ x, const voi
   float ss[TT];  // NORM: this lane's sum of x^2 of its token (row r of token tile j)
 #pragma unroll
   for (int j = 0; j < TT; ++j) ss[j] = 0.0f;
-  if constexpr (STAGED) {
-    static_assert(TT == 1 && W == 8, "staged: 8-wave, one-token-tile launches");
-    constexpr int kWTile = I8 ? 512 : 1024;               // 16 rows x 32 columns
-    constexpr int kStage = NA * RT * kWTile + 2048;        // + 16 tokens x 32 floats
-    constexpr int kPerStage = NA * RT + 2;                 // DMA instructions per stage
-    extern __shared__ __align__(16) unsigned char dyn[];
-    // [0, nbytes): the norm weight (NORM); then each wave's two stages.
-    const int nbytes = NORM ? cols * 4 : 0;
-    unsigned char* const stages = dyn + nbytes + wave * 2 * kStage;
-    const unsigned stages_lds = lds_address(stages);
-    // DMA sources. Weight tile: bf16, lane l takes row l/4, 16-byte piece
-    // (l%4) ^ (row/2 % 4); int8, lanes 0-31, row l/2, piece (l%2) ^ (row/4 % 2).
-    // Activation tile: lane l of DMA u takes token 8u + l/8, piece (l%8) ^ (l/8).
-    // LDS slot = lane, so each row's pieces land swizzled and the operand reads
-    // below spread over the banks.
-    const int wr = I8 ? (lane >> 1) : (lane >> 2);
-    const int wp = I8 ? ((lane & 1) ^ ((wr >> 2) & 1)) : ((lane & 3) ^ ((wr >> 1) & 3));
-    const char* wsrc[NA][RT];
-#pragma unroll
-    for (int i = 0; i < RT; ++i) {
-      const size_t off = (size_t(min(row0 + 16 * i + (wr & 15), rows - 1)) * cols + 8 * (I8 ? 2 : 1) * wp) *
-                         (I8 ? 1 : 2);
-      wsrc[0][i] = static_cast<const char*>(w) + off;
-      if constexpr (GATE) wsrc[NA - 1][i] = static_cast<const char*>(w2) + off;
-    }
-    const int xq = (lane & 7) ^ ((lane >> 3) & 7);
-    const float* xsrc0 = x + size_t(min(tok0 + (lane >> 3), T - 1)) * cols + 4 * xq;
-    const float* xsrc1 = x + size_t(min(tok0 + 8 + (lane >> 3), T - 1)) * cols + 4 * xq;
-    const int nblk = cols > 32 * wave ? (cols - 32 * wave + 32 * W - 1) / (32 * W) : 0;
-    auto issue = [&](const int slot, const int j) {
-      const int kb = min(32 * (wave + W * j), cols - 32);  // j < nblk: always in bounds
-      const unsigned dst = stages_lds + slot * kStage;
-#pragma unroll
-      for (int n = 0; n < NA; ++n)
-#pragma unroll
-        for (int i = 0; i < RT; ++i) {
-          const char* src = wsrc[n][i] + size_t(kb) * (I8 ? 1 : 2);
-          if constexpr (I8) {
-            if (lane < 32) dma16(src, dst + (n * RT + i) * kWTile);
-          } else {
-            dma16(src, dst + (n * RT + i) * kWTile);
-          }
-        }
-      dma16(xsrc0 + kb, dst + NA * RT * kWTile);
-      dma16(xsrc1 + kb, dst + NA * RT * kWTile + 1024);
-    };
-    // Operand offsets in a stage (the inverse of the swizzles above).
-    const int aoff = I8 ? 16 * (2 * r + ((g >> 1) ^ ((r >> 2) & 1))) + 8 * (g & 1)
-                        : 16 * (4 * r + (g ^ ((r >> 1) & 3)));
-    const int boff0 = NA * RT * kWTile + 16 * (8 * r + ((2 * g) ^ (r & 7)));
-    const int boff1 = NA * RT * kWTile + 16 * (8 * r + ((2 * g + 1) ^ (r & 7)));
-    // Blocks 0 and 1 go out first. NORM: then the norm weight, also by DMA (so
-    // that every wait here is on this wave's own count of DMAs), and the whole
-    // workgroup waits for it: its round trip overlaps the blocks' instead of
-    // preceding them.
-    if (nblk > 0) issue(0, 0);
-    if (nblk > 1) issue(1, 1);
-    if constexpr (NORM) {
-      const int n4 = cols / 4;  // 16-byte pieces; lane l of a DMA lands at base + 16 l
-      const unsigned norm_lds = lds_address(dyn);
-      for (int i0 = 64 * wave; i0 < n4; i0 += 64 * W)
-        if (i0 + lane < n4) dma16(norm.weight + 4 * (i0 + lane), norm_lds + 16 * i0);
-      wait_vmcnt<0>();
-      __syncthreads();
-    }
-    for (int j = 0; j < nblk; ++j) {
-      // Block j's tiles have landed (block j + 1's, when there is one, may not).
-      if (j + 1 < nblk)
-        wait_vmcnt<kPerStage>();
-      else
-        wait_vmcnt<0>();
-      const unsigned char* st = stages + (j & 1) * kStage;
-      float4 x0 = *reinterpret_cast<const float4*>(st + boff0);
-      float4 x1 = *reinterpret_cast<const float4*>(st + boff1);
-      if constexpr (NORM) {
-        const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-#pragma unroll
-        for (int e = 0; e < 8; ++e) ss[0] = __builtin_fmaf(v[e], v[e], ss[0]);
-        const float* wn = reinterpret_cast<const float*>(dyn) + 32 * (wave + W * j) + 8 * g;
-        const float4 wn0 = *reinterpret_cast<const float4*>(wn);
-        const float4 wn1 = *reinterpret_cast<const float4*>(wn + 4);
-        x0 = make_float4(x0.x * wn0.x, x0.y * wn0.y, x0.z * wn0.z, x0.w * wn0.w);
-        x1 = make_float4(x1.x * wn1.x, x1.y * wn1.y, x1.z * wn1.z, x1.w * wn1.w);
-      }
-      bf16x8 bh, bm, bl;
-      split3(x0, x1, bh, bm, bl);
-#pragma unroll
-      for (int n = 0; n < NA; ++n)
-#pragma unroll
-        for (int i = 0; i < RT; ++i) {
-          bf16x8 a;
-          if constexpr (I8) {
-            const uint2 raw = *reinterpret_cast<const uint2*>(st + (n * RT + i) * kWTile + aoff);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              const uint32_t word = e < 4 ? raw.x : raw.y;
-              a[e] = static_cast<bf16>(static_cast<float>(static_cast<int8_t>((word >> (8 * (e & 3))) & 0xFF)));
-            }
-          } else {
-            a = *reinterpret_cast<const bf16x8*>(st + (n * RT + i) * kWTile + aoff);
-          }
-          acc[n][i][0] = mma3(a, bh, bm, bl, acc[n][i][0]);
-        }
-      // Block j + 2 into the stage just read, once those LDS reads are done
-      // (s_waitcnt lgkmcnt(0), the other counters at their no-wait maxima).
-      if (j + 2 < nblk) {
-        __builtin_amdgcn_s_waitcnt(0xC07F);
-        issue(j & 1, j + 2);
-      }
-    }
-  } else
   for (int kb = 32 * wave; kb < cols; kb += 32 * W) {
     const int k = kb + 8 * g;
     const bool kin = k < cols;
@@ -424,44 +263,118 @@ int check_matrix(const ie_matrix& m, const char* who) {
   return IE_HIP_OK;
 }
 
-// The staged kernel's launch: dynamic LDS = the norm weight (NORM) + two stages
-// for each of the 8 waves. Returns false (nothing launched) when that exceeds
-// kStagedMaxLds; *rc is the launch status otherwise.
-constexpr int kStagedMaxLds = 128 * 1024;
+// The LDS-tiled kernel's launch. A tile shape is chosen by the time its launch should take:
+// rounds over the compute units times a workgroup's time, which is a fixed part plus a part
+// per K block of a slot. The parts (ns) were fitted on an MI355X to o_proj (896 x 896) and
+// down (896 x 4,864) with at most one workgroup per compute unit, launch overhead taken
+// off; the choice was then within 8% of the fastest shape for q/k/v, o_proj, gate/up and
+// down at 21 batch sizes from 1 to 4,000 tokens. What the shapes gain over one 16- or
+// 32-row tile per workgroup at every size (us, bf16): gate/up 16.3 -> 12.1 at 64 tokens,
+// 104 -> 44 at 600, 630 -> 252 at 4,000; down 11.1 -> 8.7, 47 -> 27, 246 -> 123.
+struct Tile {
+  int nr, ct, w;           // row tiles (of all weight matrices) and token tiles, waves
+  int fixed_ns, block_ns;  // a workgroup's time: fixed + block * (K blocks of a slot)
+};
+constexpr Tile kPlainTiles[] = {{1, 1, 8, 600, 280},  {2, 1, 8, 750, 390},  {2, 2, 8, 700, 620},
+                                {3, 2, 4, 1300, 900}, {4, 2, 4, 1600, 940}, {6, 2, 4, 2000, 1210},
+                                {8, 2, 4, 2500, 1470}};
+constexpr Tile kGateTiles[] = {{2, 1, 8, 750, 390}, {4, 1, 8, 700, 680}, {4, 2, 8, 1000, 850},
+                               {6, 2, 4, 2000, 1210}, {8, 2, 4, 2500, 1470}};
+constexpr int kTiledMaxLds = 160 * 1024;  // a gfx950 compute unit's LDS
 
-template <bool G, int R, bool I8, bool N>
-bool launch_staged_variant(const dim3 grid, hipStream_t stream, float* y, const float* x,
-                           const ie_matrix& w, const void* w2d, const float* s2, const float* bias,
-                           int T, int accumulate, RowSplit split, RowNorm norm, int* rc) {
-  constexpr int kStage = (G ? 2 : 1) * R * (I8 ? 512 : 1024) + 2048;
-  const size_t lds = (N ? size_t(w.cols) * 4 : 0) + size_t(2 * kMmWaves) * kStage;
-  if (lds > size_t(kStagedMaxLds)) return false;
-  const void* kernel = reinterpret_cast<const void*>(matmul_mfma_kernel<G, R, 1, kMmWaves, I8, N, true>);
-  if (lds > 64 * 1024) {  // above the default dynamic-LDS cap, within gfx950's 160 KB
-    static const hipError_t attr =
-        hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kStagedMaxLds);
-    if ((*rc = check_hip(attr, "hipFuncSetAttribute(matmul)"))) return true;
-  }
-  hipLaunchKernelGGL((matmul_mfma_kernel<G, R, 1, kMmWaves, I8, N, true>), grid, dim3(64 * kMmWaves),
-                     lds, stream, y, x, w.data, w.scale, w2d, s2, bias, T, w.rows, w.cols, accumulate,
-                     split, norm);
-  *rc = IE_HIP_OK;
-  return true;
-}
+// One launch of a tile shape; false (nothing launched) where its LDS or its grid does not fit.
+struct TiledLaunch {
+  float* y;
+  const float* x;
+  const ie_matrix* w;
+  const ie_matrix* w2;
+  const float* bias;
+  int T, accumulate;
+  RowSplit split;
+  RowNorm norm;
+  int vec;
+  hipStream_t stream;
 
-template <bool G, int R>
-bool launch_staged_rt(bool i8, bool n, const dim3 grid, hipStream_t stream, float* y,
-                      const float* x, const ie_matrix& w, const void* w2d, const float* s2,
-                      const float* bias, int T, int accumulate, RowSplit split, RowNorm norm,
-                      int* rc) {
-#define IE_MM_STAGED(I, N_)                                                                    return launch_staged_variant<G, R, I, N_>(grid, stream, y, x, w, w2d, s2, bias, T, accumulate,                                             split, norm, rc)
-  if (i8) {
-    if (n) IE_MM_STAGED(true, true);
-    IE_MM_STAGED(true, false);
+  template <bool GATE, int NR, int CT, int W, int SLOTS, int S, bool I8, bool NORM>
+  bool go(int* rc) const {
+    constexpr int RT = NR / (GATE ? 2 : 1);
+    using Shape = TiledShape<GATE, RT, CT, W, S, I8>;
+    const int64_t lds = int64_t(Shape::kLds) + (NORM ? int64_t(w->cols) * 4 : 0);
+    const int64_t row_tiles = (int64_t(w->rows) + Shape::kRows - 1) / Shape::kRows;
+    const int64_t tok_tiles = (int64_t(T) + Shape::kTokens - 1) / Shape::kTokens;
+    if (lds > kTiledMaxLds || row_tiles * tok_tiles * 64 * W > int64_t(UINT32_MAX)) return false;
+    const auto kernel = matmul_tiled_kernel<GATE, RT, CT, W, SLOTS, S, I8, NORM>;
+    if (lds > 64 * 1024) {  // above the default dynamic-LDS cap
+      static const hipError_t attr =
+          hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, kTiledMaxLds);
+      if ((*rc = check_hip(attr, "hipFuncSetAttribute(matmul)"))) return true;
+    }
+    hipLaunchKernelGGL(kernel, dim3(unsigned(row_tiles * tok_tiles)), dim3(64 * W), unsigned(lds),
+                       stream, y, x, w->data, w->scale, w2 ? w2->data : nullptr,
+                       w2 ? w2->scale : nullptr, bias, T, w->rows, w->cols, accumulate, split, norm,
+                       vec, int(row_tiles), int(tok_tiles));
+    *rc = IE_HIP_OK;
+    return true;
   }
-  if (n) IE_MM_STAGED(false, true);
-  IE_MM_STAGED(false, false);
-#undef IE_MM_STAGED
+  template <bool GATE, int NR, int CT, int W, int SLOTS, int S>
+  bool with_types(int* rc) const {
+    if constexpr (SLOTS == 8) {  // the folded rmsnorm: matrices below 16 row tiles per unit
+      if (norm.weight)
+        return w->int8 ? go<GATE, NR, CT, W, SLOTS, S, true, true>(rc)
+                       : go<GATE, NR, CT, W, SLOTS, S, false, true>(rc);
+    }
+    return w->int8 ? go<GATE, NR, CT, W, SLOTS, S, true, false>(rc)
+                   : go<GATE, NR, CT, W, SLOTS, S, false, false>(rc);
+  }
+  template <bool GATE>
+  bool run(int shape, int* rc) const {
+    if constexpr (GATE) {
+      switch (shape) {
+        case 0: return with_types<true, 2, 1, 8, 8, 2>(rc);
+        case 1: return with_types<true, 4, 1, 8, 8, 1>(rc);
+        case 2: return with_types<true, 4, 2, 8, 8, 1>(rc);
+        case 3: return with_types<true, 6, 2, 4, 8, 1>(rc);
+        default: return with_types<true, 8, 2, 4, 8, 1>(rc);
+      }
+    } else {
+      switch (shape) {
+        case 0: return with_types<false, 1, 1, 8, 8, 2>(rc);
+        case 1: return with_types<false, 2, 1, 8, 8, 1>(rc);
+        case 2: return with_types<false, 2, 2, 8, 8, 1>(rc);
+        case 3: return with_types<false, 3, 2, 4, 8, 1>(rc);
+        case 4: return with_types<false, 4, 2, 4, 8, 1>(rc);
+        case 5: return with_types<false, 6, 2, 4, 8, 1>(rc);
+        default: return with_types<false, 8, 2, 4, 8, 1>(rc);
+      }
+    }
+  }
+  // Wide matrices (4 slots, one wave each). The 151,936-row LM head, us: at 1 to 16 tokens 64
+  // rows x 16 tokens is the best shape (1 token, bf16: 59 before, 52; INT8: 60 -> 38), from
+  // 17 on 128 x 32 (64 tokens, bf16: 138 -> 92, INT8: 177 -> 74).
+  bool run_wide(bool gate, int* rc) const {
+    if (gate) return with_types<true, 8, 2, 4, 4, 1>(rc);
+    return T <= 16 ? with_types<false, 4, 1, 4, 4, 2>(rc) : with_types<false, 8, 2, 4, 4, 1>(rc);
+  }
+};
+
+int choose_tile(bool gate, int rows, int cols, int T, int cus) {
+  const Tile* tiles = gate ? kGateTiles : kPlainTiles;
+  const int count = gate ? int(std::size(kGateTiles)) : int(std::size(kPlainTiles));
+  const int64_t blocks = (cols / 32 + 7) / 8;
+  int best = 0;
+  int64_t best_ns = INT64_MAX;
+  for (int i = 0; i < count; ++i) {
+    const Tile& t = tiles[i];
+    const int64_t rt = 16 * (gate ? t.nr / 2 : t.nr), tt = 16 * t.ct;
+    const int64_t groups = ((rows + rt - 1) / rt) * ((T + tt - 1) / tt);
+    const int64_t ns = ((groups + cus - 1) / cus) * (t.fixed_ns + t.block_ns * blocks);
+    if (ns < best_ns) {
+      best_ns = ns;
+      best = i;
+    }
+  }
+  return best;
 }
 
 int launch_matmul(bool gate, float* y, const float* x, const ie_matrix& w, const ie_matrix* w2,
@@ -484,63 +397,54 @@ int launch_matmul(bool gate, float* y, const float* x, const ie_matrix& w, const
                           (w2 ? reinterpret_cast<uintptr_t>(w2->data) : 0);
   if (align & (w.int8 ? 7 : 15))
     return fail(IE_HIP_EINVAL, std::string(who) + ": x and the weights must be 16-byte aligned");
-  // The waves of a workgroup split K, so their count fixes every output's
-  // summation order. It depends on the matrix alone, never on T: a token's
-  // result is then the same bit for bit whatever batch it is computed in (the
-  // reference's "batch of N == N single tokens" contract,
-  // src/cuda/cuda_runner.cu:798-829). Wide matrices (row tiles alone reach 16
-  // per compute unit: the 151,936-row LM head) take 4-wave workgroups of 4 x 4
-  // tiles: at ~140 registers a lane three fit on a compute unit where one of 8
-  // would (LM head at 64 tokens: 176 -> 149 us on MI355X), each weight is read
-  // once and each activation fragment a quarter as often (366 -> 172 us).
-  // Otherwise 8 waves, and the tiles per workgroup (which do not change the
-  // arithmetic) follow the count of 16 x 16 output tiles, measured at 64
-  // tokens: below 4 per compute unit (q/k/v/o and down at 896 rows) one tile
-  // per workgroup keeps every unit busy; from 4 per unit two row tiles share
-  // each activation fragment, except for gate/up in the staged kernel (one row
-  // tile, below).
+  // K is split over slots whose count fixes every output's summation order. It depends on
+  // the matrix alone, never on T: a token's result is then the same bit for bit whatever
+  // batch it is computed in (the reference's "batch of N == N single tokens" contract,
+  // src/cuda/cuda_runner.cu:798-829): 4 for wide matrices (row tiles alone reach 16 per
+  // compute unit: the 151,936-row LM head), where fewer, longer waves fill the chip, else 8.
   const int cus = device_compute_units();
   const bool wide = (w.rows + 15) / 16 >= 16 * cus;
   const int waves = wide ? 4 : kMmWaves;
-  const int64_t tiles = int64_t((w.rows + 15) / 16) * ((T + 15) / 16);
-  int RT = wide ? 4 : tiles >= 4 * int64_t(cus) ? 2 : 1;
-  // The staged kernel (below) for every 8-wave launch whose K is whole 32-column
-  // blocks and whose weights are 16-byte aligned (for the DMA).
-  const bool staged = !wide && w.cols % 32 == 0 &&
-                      ((reinterpret_cast<uintptr_t>(w.data) |
-                        reinterpret_cast<uintptr_t>(w2 ? w2->data : nullptr)) & 15) == 0;
-  // Two weight matrices: at most 2 row tiles; staged, one (its LDS then fits two
-  // workgroups on a compute unit: config 6's gate/up, 1.657 -> 1.608 ms a step).
-  if (gate) RT = std::min(RT, staged ? 1 : 2);
+  if (norm.weight && wide)
+    return fail(IE_HIP_EINVAL, std::string(who) + ": too many rows for the folded rmsnorm");
   const int tok_tiles = (T + 15) / 16;  // kernels exist for 1, 2 and 4 token tiles
   const int TT = !wide ? 1 : tok_tiles > 2 ? 4 : tok_tiles;
-  const dim3 grid((w.rows + 16 * RT - 1) / (16 * RT), (T + 16 * TT - 1) / (16 * TT));
-  const dim3 block(64 * waves);
-  if (grid.y > 65535) return fail(IE_HIP_EINVAL, std::string(who) + ": too many tokens");
-  const void* w2d = gate ? w2->data : nullptr;
-  const float* s2 = gate ? w2->scale : nullptr;
-  // The staged kernel: the same operands in the same order, so the same results
-  // as the direct loads below.
-  if (staged) {
+  if ((T + 16 * TT - 1) / (16 * TT) > 65535)
+    return fail(IE_HIP_EINVAL, std::string(who) + ": too many tokens");
+  // LDS tiles: K in whole 32-wide blocks, at least one per slot, and 16-byte aligned weights
+  // for the DMA (x always is).
+  const uintptr_t weights = reinterpret_cast<uintptr_t>(w.data) |
+                            reinterpret_cast<uintptr_t>(w2 ? w2->data : nullptr);
+  if (w.cols % 32 == 0 && w.cols >= 32 * waves && ((reinterpret_cast<uintptr_t>(x) | weights) & 15) == 0) {
+    const uintptr_t out = reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(split.y1) |
+                          reinterpret_cast<uintptr_t>(split.y2) | reinterpret_cast<uintptr_t>(bias) |
+                          reinterpret_cast<uintptr_t>(w.scale) |
+                          reinterpret_cast<uintptr_t>(w2 ? w2->scale : nullptr);
+    const int vec = (out & 15) == 0 && ((w.rows | split.split0 | split.split1) & 3) == 0;
+    const TiledLaunch launch{y, x, &w, w2, bias, T, accumulate, split, norm, vec, stream};
     int rc = IE_HIP_OK;
-    const bool n = norm.weight != nullptr;
     bool launched;
-    if (gate)
-      launched = RT == 2 ? launch_staged_rt<true, 2>(w.int8, n, grid, stream, y, x, w, w2d, s2, bias,
-                                                     T, accumulate, split, norm, &rc)
-                         : launch_staged_rt<true, 1>(w.int8, n, grid, stream, y, x, w, w2d, s2, bias,
-                                                     T, accumulate, split, norm, &rc);
-    else
-      launched = RT == 2 ? launch_staged_rt<false, 2>(w.int8, n, grid, stream, y, x, w, w2d, s2, bias,
-                                                      T, accumulate, split, norm, &rc)
-                         : launch_staged_rt<false, 1>(w.int8, n, grid, stream, y, x, w, w2d, s2, bias,
-                                                      T, accumulate, split, norm, &rc);
+    if (wide) {
+      launched = launch.run_wide(gate, &rc);
+    } else {
+      const int shape = choose_tile(gate, w.rows, w.cols, T, cus);
+      launched = gate ? launch.run<true>(shape, &rc) : launch.run<false>(shape, &rc);
+      // A folded rmsnorm's weights can leave too little LDS for the shape: the smallest one.
+      if (!launched && shape != 0)
+        launched = gate ? launch.run<true>(0, &rc) : launch.run<false>(0, &rc);
+    }
     if (launched) return rc != IE_HIP_OK ? rc : check_launch(who);
   }
+  // Direct loads. Tiles per workgroup from the count of 16 x 16 output tiles: two row tiles
+  // from 4 per compute unit on, 4 x 4 (or the token tiles there are) for wide matrices.
+  const int64_t tiles = int64_t((w.rows + 15) / 16) * tok_tiles;
+  int RT = wide ? 4 : tiles >= 4 * int64_t(cus) ? 2 : 1;
+  if (gate) RT = std::min(RT, 2);
+  const dim3 grid((w.rows + 16 * RT - 1) / (16 * RT), (T + 16 * TT - 1) / (16 * TT));
+  const dim3 block(64 * waves);
+  const void* w2d = gate ? w2->data : nullptr;
+  const float* s2 = gate ? w2->scale : nullptr;
   if (norm.weight) {
-    // The folded rmsnorm exists for the 8-wave, one-token-tile launches (every
-    // matrix below 16 row tiles per compute unit).
-    if (wide) return fail(IE_HIP_EINVAL, std::string(who) + ": too many rows for the folded rmsnorm");
 #define IE_MM_NORM(G, R)                                                                          \
   do {                                                                                            \
     if (w.int8)                                                                                   \

@@ -286,3 +286,52 @@ def test_dense_argument_errors(ie, dev):
     w2 = torch.zeros((8, 16), dtype=torch.int16, device=dev)
     with pytest.raises(ie.IeHipError, match="shapes differ"):
         ie.gate_up_silu(y, torch.zeros((4, 16), device=dev), ie.matrix(w1), ie.matrix(w2))
+
+
+# T, rows, cols: every LDS tile shape with ragged edges (rows % 16, rows % 4, T % 16 and the K
+# blocks' share per slot all uneven), the smallest K that takes LDS tiles and the one below it.
+TILED = [(1, 898, 288), (17, 898, 288), (77, 898, 288), (200, 898, 288), (333, 898, 288),
+         (600, 898, 288), (1003, 898, 288), (450, 1152, 896), (50, 900, 256), (50, 900, 224),
+         (9, 70001, 128), (21, 70001, 160)]
+
+
+@pytest.mark.parametrize("T,rows,cols", TILED)
+@pytest.mark.parametrize("int8", [False, True])
+def test_tile_shapes(ie, dev, T, rows, cols, int8):
+    """Against the oracle (float32 rounding of the sums), and the first and last token bit for
+    bit what they are alone, whatever tile shape the batch took."""
+    rng = np.random.default_rng(T + rows + cols)
+    x = rng.standard_normal((T, cols), dtype=np.float32)
+    w32 = rng.standard_normal((rows, cols), dtype=np.float32) * np.float32(0.05)
+    m, keep, (w, fmt, s) = dev_weights(ie, dev, w32, int8)
+    dx = torch.from_numpy(x).to(dev)
+    y = torch.full((T, rows), float("nan"), device=dev)
+    ie.matmul(y, dx, m)
+    one = torch.empty((1, rows), device=dev)
+    torch.cuda.synchronize()
+    assert rel_err(y.cpu().numpy(), O.matmul(x, w, fmt, s, None)) <= REL
+    for t in (0, T - 1):
+        ie.matmul(one, dx[t:t + 1].contiguous(), m)
+        torch.cuda.synchronize()
+        assert torch.equal(one[0].view(torch.int32), y[t].view(torch.int32)), t
+
+
+@pytest.mark.parametrize("T", [1, 20, 40, 90, 300])
+@pytest.mark.parametrize("int8", [False, True])
+def test_gate_tile_shapes(ie, dev, T, int8):
+    """The gate/up form of each shape, with and without the folded rmsnorm, at 4,866 rows."""
+    rng = np.random.default_rng(T)
+    rows, cols = 4866, 288
+    x = rng.standard_normal((T, cols), dtype=np.float32)
+    ws = [dev_weights(ie, dev, rng.standard_normal((rows, cols), dtype=np.float32) * np.float32(0.1),
+                      int8) for _ in range(2)]
+    wn = rng.standard_normal(cols, dtype=np.float32)
+    dx, dn = torch.from_numpy(x).to(dev), torch.from_numpy(wn).to(dev)
+    for xin, call in ((x, lambda o: ie.gate_up_silu(o, dx, ws[0][0], ws[1][0])),
+                      (O.rmsnorm(x, wn, 1e-6),
+                       lambda o: ie.rmsnorm_gate_up_silu(o, dx, dn, 1e-6, ws[0][0], ws[1][0]))):
+        out = torch.full((T, rows), float("nan"), device=dev)
+        call(out)
+        torch.cuda.synchronize()
+        g, u = (O.matmul(xin, w, fmt, s, None) for _, _, (w, fmt, s) in ws)
+        assert rel_err(out.cpu().numpy(), O.silu_mul(g, u)) <= REL
