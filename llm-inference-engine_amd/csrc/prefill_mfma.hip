@@ -1,6 +1,6 @@
 // Chunked-prefill attention into pages on the matrix cores (gfx950), for KV
-// caches of every type with head_dim 64: 16-bit caches on the 16-bit
-// instructions (prefill_mfma_kernel), f32 caches on the f32 ones
+// caches of every type with head_dim 64: 16-bit caches in their own type
+// (prefill_mfma_kernel), f32 caches in three bf16 parts
 // (prefill_mfma_f32_kernel, further down).
 //
 // Reference semantics: each row's causal GQA attention over positions
@@ -54,6 +54,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "matmul_tiled.hpp"
 #include "mfma.hpp"
 #include "prefill.hpp"
 
@@ -685,270 +686,313 @@ int launch_prefill_mfma(float* out, const float* q, const uint16_t* kp, const ui
 
 
 // ---------------------------------------------------------------------------
-// float32 KV caches: the same block structure on v_mfma_f32_16x16x4_f32 (full
-// fp32 operands: no hi + lo split, 16x the matrix-core time per product of the
-// 16-bit kernel, still far above the VALU path).
-//   S^T[16 keys x 16 rows] per key group of 16: 16 steps of 4 dims; step s
-//     takes dims 16g + s for lane group g, so lane (g, r) reads key r's dims
-//     16g .. 16g+15 (64 bytes, 4 LDS reads) and holds, as B, row r's query at
-//     the same dims.
-//   O^T[64 dims x 16 rows] += V^T . P^T: 16 steps of 4 keys; step (kt4, s)
-//     takes keys 16 kt4 + 4g + s, so lane (g, r)'s B operand is its own score
-//     of that key; row i of tile mt is dim 4i + mt, so its A operand is the
-//     16-byte piece r of that key's V row (one LDS read, the 4 tiles' values).
-//     Lane (g, r) ends up holding row r's dims 16g + 4t + mt (o[mt][t]).
-// K/V tiles of 64 keys (16 KB each, f32) go through a ring of 3 tiles in LDS
-// by DMA. K rows are stored with their 16-byte pieces swizzled (piece ^ (key
-// & 15)), so the 16 lanes of a group reading the same dims of 16 keys hit
-// distinct banks; V rows are read a whole row per 16 lanes and stay as they are.
-constexpr int kTileF32 = kKeys * 64 * 4;     // 16 KB: one f32 K or V tile of one KV head
-constexpr int kBufF32 = 2 * kTileF32;        // K tile + V tile
-constexpr int kRingF32 = 3;
+// float32 KV caches. Queries, keys, weights and values enter the 16-bit matrix cores in
+// three bf16 parts each, x = hi + mid + lo exactly (split3), and every product is the six
+// largest of the nine partial ones: what is left out is below 2^-26 of the product, under
+// the rounding of its float32 sum. (Measured against float64: 4.4e-7 at 1,333 rows on 1,000
+// cached, where v_mfma_f32_16x16x4_f32 on the whole float32 values gave 8.0e-7.) The f32
+// instruction takes 256 cycles for the 16x16x32 product that six bf16 ones do in 96, and no
+// VALU instruction runs beside it (probe: 52 cycles with four VALU instructions beside it,
+// 35 alone), while the bf16 ones leave the VALU free for the splits and the softmax.
+//
+// One workgroup per (NB blocks of 16 rows, query head); its waves take 32-key tiles in turn,
+// each with its own K stage, softmax state and output, merged through LDS at the end: no
+// barrier and no sharing until then, and T / 16 / NB x heads workgroups, the longest
+// contexts first, where a workgroup per pair of blocks and KV head left two thirds of the
+// compute units idle at 1,333 rows. What bounds it now is VALU issue: a tile's K and V take
+// 352 instructions to split, shared by NB blocks. Times (us, was 7 waves on shared f32
+// tiles): 1,333 rows on 1,000 cached 237 -> 73, 4,000 rows 281 -> 194, 130 rows on 4,000
+// cached 548 -> 44.
+//   S^T[16 keys x 16 rows] per key group of 16: step ks takes dims 16g + 8ks .. +7, so lane
+//     (g, r) reads key r's dims 16g .. 16g+15 (64 bytes, 4 LDS reads).
+//   O^T[64 dims x 16 rows] += V^T . P^T: one step of 32 keys; lane (g, r)'s B operand is its
+//     own 8 weights, keys 16 kt + 4g + e; row i of tile mt is dim 4i + mt, so its A operand
+//     is one component of the 16-byte pieces r of those keys' V rows: 16 lanes read a whole
+//     256-byte row, so V comes straight from memory into registers, sent for before the
+//     scores and used after the softmax. Lane (g, r) ends up with row r's dims
+//     16g + 4t + mt (o[mt][t]).
+// K tiles (8 KB) come through LDS by DMA, one stage per wave: read whole into registers,
+// then the next tile is sent for. K rows are stored with their 16-byte pieces swizzled
+// (piece ^ (key & 15)), so the 16 lanes of a group reading the same dims of 16 keys hit
+// distinct banks.
+constexpr int kKeysF32 = 32;                      // keys per wave tile (2 pages)
+constexpr int kStageF32 = kKeysF32 * 64 * 4;      // 8 KB of K
+// The six products of two operands in three parts (0 the largest), the smallest first.
+__device__ constexpr int kPartA[6] = {2, 0, 1, 1, 0, 0};
+__device__ constexpr int kPartB[6] = {0, 2, 1, 0, 1, 0};
 
-template <int kWaves>
-__global__ void __launch_bounds__(64 * kWaves)
+template <int NB, int kTeams>
+__global__ void __launch_bounds__(64 * kTeams)
 prefill_mfma_f32_kernel(float* __restrict__ out, const float* __restrict__ q,
                         const float* __restrict__ k_pool, const float* __restrict__ v_pool, int T,
                         const int32_t* __restrict__ row_pos, const int32_t* __restrict__ row_seq,
                         const int32_t* __restrict__ tables, int max_pages, int num_pages,
-                        int n_heads, int n_kv_heads, int n_blocks) {
-  // A tile's 32 loads of 1 KB (16 K, 16 V), spread evenly over kDmaWaves waves.
-  constexpr int kDmaWaves = kWaves >= 4 ? 4 : kWaves >= 2 ? 2 : 1;
-  constexpr int kPerWave = 32 / kDmaWaves;
-  extern __shared__ __align__(16) unsigned char smem[];
+                        int n_heads, int n_kv_heads, int n_units) {
+  // The K stages; at the end each wave's (o, m, l).
+  constexpr int kMergeF32 = kTeams * NB * (4 * 1024 + 512);
+  __shared__ __align__(16) unsigned char smem[kTeams * kStageF32 > kMergeF32
+                                                  ? kTeams * kStageF32 : kMergeF32];
   const int group = n_heads / n_kv_heads;
-  const int kvh = blockIdx.y;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, r = lane & 15;
-  const int h0 = kvh * group + wave;  // this wave's head
+  // Workgroups go to the 8 XCDs in turn. Where the KV heads divide 8, an XCD takes one KV
+  // head's work only, so its L2 holds that head's K and V.
+  const int spread = 8 % n_kv_heads == 0 ? 8 / n_kv_heads : 1;  // XCDs per KV head
+  int kvh, unit;
+  if (8 % n_kv_heads == 0) {
+    kvh = (blockIdx.x & 7) % n_kv_heads;
+    unit = int(blockIdx.x >> 3) * spread + (blockIdx.x & 7) / n_kv_heads;
+  } else {
+    kvh = blockIdx.x % n_kv_heads;
+    unit = blockIdx.x / n_kv_heads;
+  }
+  if (unit >= n_units * group) return;
+  const int block = n_units - 1 - unit / group;  // longest contexts first
+  const int head = kvh * group + unit % group;
   const int kv_dim = n_kv_heads * 64;
   const int pos0 = __builtin_amdgcn_readfirstlane(row_pos[0]);
   const int seq = __builtin_amdgcn_readfirstlane(row_seq[0]);
   const int32_t* tab = tables + size_t(seq) * max_pages;
-  // Page ids of a segment of key tiles staged in LDS after the ring, as in the
-  // 16-bit kernel: ids[4 (tile - seg0) + j], -1 past the table row or outside
-  // the pool.
-  int* const ids = reinterpret_cast<int*>(smem + kRingF32 * kBufF32);
-  int seg0 = 0;
-  auto tile_ids = [&](const int tile) {
-    return *reinterpret_cast<const int4*>(ids + 4 * (tile - seg0));
-  };
-  auto tile_ok = [&](const int tile) -> int {
-    const int4 v = tile_ids(tile);
-    return __builtin_amdgcn_readfirstlane(int(v.x >= 0) | (int(v.y >= 0) << 1) |
-                                          (int(v.z >= 0) << 2) | (int(v.w >= 0) << 3));
-  };
+  const int t0 = block * 16 * NB;
+  const int max_pos = pos0 + min(t0 + 16 * NB, T) - 1;  // last position any row sees
+  const int min_pos = pos0 + t0;
+  const int n_tiles = max_pos / kKeysF32 + 1;
 
-  // DMA of a tile into buffer `buf`: load u (0..15 K, 16..31 V) moves keys
-  // 4 (u & 15) .. +3 (page (u & 15) / 4 of the tile); lane l lands at base + 16 l:
-  // key 4 (u & 15) + l / 16, LDS slot l % 16, holding global piece slot ^ (key & 15)
-  // for K and piece slot for V.
+  // Row r's query of each block, times log2(e)/8, in three parts: B of the scores' step ks is
+  // dims 16g + 8ks .. +7.
+  bf16x8 qp[NB][2][3];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const int t = t0 + 16 * b + r;
+    const float4* src =
+        reinterpret_cast<const float4*>(q + (size_t(t < T ? t : t0) * n_heads + head) * 64 + 16 * g);
+    const float qs = t < T ? 0.125f * kLog2e : 0.0f;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const float4 x = src[2 * ks], y = src[2 * ks + 1];
+      split3(make_float4(x.x * qs, x.y * qs, x.z * qs, x.w * qs),
+             make_float4(y.x * qs, y.y * qs, y.z * qs, y.w * qs), qp[b][ks][0], qp[b][ks][1],
+             qp[b][ks][2]);
+    }
+  }
+
+  // Page ids of a tile, -1 past the table row or outside the pool.
+  auto page = [&](int at) {
+    const int id = at < max_pages ? tab[at] : -1;
+    return __builtin_amdgcn_readfirstlane(id >= 0 && id < num_pages ? id : -1);
+  };
+  // DMA of a tile's K rows: load u moves keys 4u .. 4u+3, lane l key 4u + l/16, LDS slot
+  // l % 16, holding piece slot ^ (key & 15).
   const size_t row_bytes = size_t(kv_dim) * 4;
-  const int lkey = lane >> 4, lslot = lane & 15;
-  const unsigned smem_lds = lds_address(smem);
-  const char* kbase_g = reinterpret_cast<const char*>(k_pool) + kvh * 256;
-  const char* vbase_g = reinterpret_cast<const char*>(v_pool) + kvh * 256;
-  auto issue = [&](const int buf, const int tile) {
-    if (wave >= kDmaWaves) return;
-    const int4 v = tile_ids(tile);
-    const int id0 = max(__builtin_amdgcn_readfirstlane(v.x), 0);
-    const int id1 = max(__builtin_amdgcn_readfirstlane(v.y), 0);
-    const int id2 = max(__builtin_amdgcn_readfirstlane(v.z), 0);
-    const int id3 = max(__builtin_amdgcn_readfirstlane(v.w), 0);
+  const size_t page_bytes = size_t(IE_HIP_PAGE_SIZE) * row_bytes;
+  const char* const kbase_g = reinterpret_cast<const char*>(k_pool) + kvh * 256;
+  const char* const vbase_g = reinterpret_cast<const char*>(v_pool) + kvh * 256;
+  unsigned char* const stage = smem + wave * kStageF32;
+  const unsigned stage_lds = lds_address(stage);
+  size_t koff[4], voff[4];
 #pragma unroll
-    for (int k = 0; k < kPerWave; ++k) {
-      const int u = wave * kPerWave + k;        // 0..31
-      const bool is_v = u >= 16;
-      const int uu = u & 15;
-      const int pg = uu >> 2;                   // page of the tile
-      const int id = pg == 0 ? id0 : pg == 1 ? id1 : pg == 2 ? id2 : id3;
-      const int key = 4 * uu + lkey;            // key within the tile
-      const int piece = is_v ? lslot : (lslot ^ (key & 15));
-      const char* src = (is_v ? vbase_g : kbase_g) +
-                        (size_t(id) * IE_HIP_PAGE_SIZE + (key & 15)) * row_bytes +
-                        16 * piece;
-      dma16(src, smem_lds + buf * kBufF32 + (is_v ? kTileF32 : 0) + uu * 1024);
-    }
-  };
-  auto wait_tiles = [&](const int newer) {
-    if (newer >= 1) wait_vmcnt<kPerWave>();
-    else wait_vmcnt<0>();
+  for (int u = 0; u < 4; ++u) {
+    const int key = 4 * u + g;
+    koff[u] = key * row_bytes + 16 * (r ^ key);
+    voff[u] = (4 * g + u) * row_bytes + 16 * r;
+  }
+  auto issue_k = [&](int ida, int idb) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      dma16(kbase_g + size_t(max(u < 4 ? ida : idb, 0)) * page_bytes + koff[u & 3],
+            stage_lds + u * 1024);
   };
 
-  for (int pass = 0; pass < 2; ++pass) {
-    const int hi_block = n_blocks - 1 - int(blockIdx.x);
-    const int rb = pass == 0 ? hi_block : int(blockIdx.x);
-    if (pass == 1 && rb == hi_block) break;  // the middle block of an odd count
-    const int t0 = rb * kRows;
-    const int t_last = min(t0 + kRows, T) - 1;
-    const int max_pos = pos0 + t_last;
-    const int min_pos = pos0 + t0;
-    const int n_tiles = max_pos / kKeys + 1;
-    const int t = t0 + r;
-    const bool row_ok = t < T;
-    const int rp = pos0 + t;
-
-    // Row r's query, times log2(e)/8, at dims 16g .. 16g+15 (B of the score steps).
-    float qb[16];
-    {
-      const float4* src = reinterpret_cast<const float4*>(
-          q + (size_t(row_ok ? t : t0) * n_heads + h0) * 64 + 16 * g);
-      const float qs = row_ok ? 0.125f * kLog2e : 0.0f;
+  float m[NB], l[NB];  // running max (base 2), this lane's part of the sum
+  f32x4 o[NB][4];      // o[b][mt][t]: row r of block b, dim 16g + 4t + mt
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float4 x = src[i];
-        qb[4 * i + 0] = x.x * qs;
-        qb[4 * i + 1] = x.y * qs;
-        qb[4 * i + 2] = x.z * qs;
-        qb[4 * i + 3] = x.w * qs;
+  for (int b = 0; b < NB; ++b) {
+    m[b] = -INFINITY;
+    l[b] = 0.0f;
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) o[b][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+
+  int id0 = -1, id1 = -1;  // the tile's pages
+  if (wave < n_tiles) {
+    id0 = page(2 * wave);
+    id1 = page(2 * wave + 1);
+    issue_k(id0, id1);
+  }
+  for (int tile = wave; tile < n_tiles; tile += kTeams) {
+    const int kbase = tile * kKeysF32;
+    const bool more = tile + kTeams < n_tiles;
+    int next0 = -1, next1 = -1;
+    if (more) {
+      next0 = page(2 * (tile + kTeams));
+      next1 = page(2 * (tile + kTeams) + 1);
+    }
+    wait_vmcnt<0>();  // the tile's K rows have landed
+    float4 ka[2][4];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        ka[kt][i] = *reinterpret_cast<const float4*>(stage + (16 * kt + r) * 256 +
+                                                     16 * ((4 * g + i) ^ r));
+    if (more) {
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the stage's reads are done
+      issue_k(next0, next1);
+    }
+    // V rows of the tile: step (kt, e) is key 16 kt + 4g + e, dims 4r .. 4r+3.
+    float4 v[2][4];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        v[kt][e] = *reinterpret_cast<const float4*>(
+            vbase_g + size_t(max(kt ? id1 : id0, 0)) * page_bytes + voff[e]);
+
+    float mref[NB];
+    f32x4 s[NB][2];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      mref[b] = m[b] == -INFINITY ? 0.0f : m[b];
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) s[b][kt] = f32x4{-mref[b], -mref[b], -mref[b], -mref[b]};
+    }
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        bf16x8 kp[3];
+        split3(ka[kt][2 * ks], ka[kt][2 * ks + 1], kp[0], kp[1], kp[2]);
+#pragma unroll
+        for (int p = 0; p < 6; ++p)
+#pragma unroll
+          for (int b = 0; b < NB; ++b)
+            s[b][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[kPartA[p]], qp[b][ks][kPartB[p]],
+                                                               s[b][kt], 0, 0, 0);
+      }
+    // Keys a row may not see, or in pages outside the pool: no weight, and V rows that
+    // nothing may see zeroed (stale or non-finite memory must not reach O through 0 * x).
+    if (kbase + kKeysF32 - 1 > min_pos || (id0 | id1) < 0) {
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        const bool ok = (kt ? id1 : id0) >= 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int kp = kbase + 16 * kt + 4 * g + e;
+#pragma unroll
+          for (int b = 0; b < NB; ++b)
+            s[b][kt][e] = ok && kp <= pos0 + t0 + 16 * b + r ? s[b][kt][e] : -INFINITY;
+          if (!ok || kp > max_pos) v[kt][e] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
       }
     }
-    float m = -INFINITY, l = 0.0f;  // running max (base 2), this lane's part of the sum
-    f32x4 o[4];                      // o[mt][t]: row r, dim 16g + 4t + mt
+    // Online softmax on s - mref, the reference max raised lazily (as in the
+    // 16-bit kernel: O and l rescaled only when a row's max grows past
+    // m + kLazyMax somewhere in the wave).
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) o[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    // Segments of kSegTiles key tiles, each with its page ids staged in LDS;
-    // within a segment, a ring of kRingF32 tiles.
-    for (seg0 = 0; seg0 < n_tiles; seg0 += kSegTiles) {
-      const int seg_end = min(n_tiles, seg0 + kSegTiles);
-      // The ring is idle and every wave is past its last read of the old ids.
-      for (int i = tid; i < 4 * (seg_end - seg0); i += 64 * kWaves) {
-        const int pi = 4 * seg0 + i;
-        const int id = pi < max_pages ? tab[pi] : -1;
-        ids[i] = id >= 0 && id < num_pages ? id : -1;
+    for (int b = 0; b < NB; ++b) {
+      float mx = max_nn(max3_nn(s[b][0][0], s[b][0][1], s[b][0][2]),
+                        max3_nn(max_nn(s[b][0][3], s[b][1][0]), s[b][1][1],
+                                max_nn(s[b][1][2], s[b][1][3])));
+      mx = group_max4(mx);
+      const bool grow = m[b] == -INFINITY ? mx != -INFINITY : mx > kLazyMax;
+      if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+        const float m_new = fmaxf(m[b], mref[b] + mx);
+        const float corr = m_new == -INFINITY ? 1.0f : exp2_weight(m[b] - m_new);  // m = -inf: 0
+        l[b] *= corr;
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) o[b][mt] *= corr;
+        m[b] = m_new;
+        const float shift = (m_new == -INFINITY ? 0.0f : m_new) - mref[b];
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) s[b][kt] -= shift;
       }
-      __syncthreads();
-      for (int pre = 0; pre < kRingF32 - 1 && seg0 + pre < seg_end; ++pre) issue(pre, seg0 + pre);
-      wait_tiles(min(kRingF32 - 2, seg_end - seg0 - 1));  // the segment's first tile has landed
-      __syncthreads();
-
-      int buf = 0, ibuf = kRingF32 - 1;
-      for (int kb = seg0; kb < seg_end; ++kb) {
-        const int ahead = kb + kRingF32 - 1;
-        if (ahead < seg_end)  // its buffer held tile kb - 1: free since the last barrier
-          issue(ibuf, ahead);
-        ibuf = ibuf + 1 == kRingF32 ? 0 : ibuf + 1;
-        const int kbase = kb * kKeys;
-        const unsigned char* kt = smem + buf * kBufF32;
-        unsigned char* vt = smem + buf * kBufF32 + kTileF32;
-        buf = buf + 1 == kRingF32 ? 0 : buf + 1;
-        const int okb = tile_ok(kb);
-        // Keys past max_pos or in pages outside the pool: zero their V rows first.
-        if (kbase + kKeys - 1 > max_pos || okb != 15) {
-          for (int i = tid; i < kKeys * 16; i += 64 * kWaves) {
-            const int key = i >> 4;
-            if (kbase + key > max_pos || !((okb >> (key >> 4)) & 1))
-              *reinterpret_cast<uint4*>(vt + key * 256 + (i & 15) * 16) = make_uint4(0, 0, 0, 0);
-          }
-          __syncthreads();
+      float sum = 0.0f;
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          s[b][kt][e] = exp2_weight(s[b][kt][e]);
+          sum += s[b][kt][e];
         }
-        const float mref = m == -INFINITY ? 0.0f : m;
-        // S^T per key group kt4: A = key 16 kt4 + r, dims 16g + s.
-        f32x4 s[4];
-#pragma unroll
-        for (int kt4 = 0; kt4 < 4; ++kt4) {
-          const int key = 16 * kt4 + r;
-          float ka[16];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float4 x = *reinterpret_cast<const float4*>(kt + key * 256 +
-                                                              16 * ((4 * g + i) ^ (key & 15)));
-            ka[4 * i + 0] = x.x;
-            ka[4 * i + 1] = x.y;
-            ka[4 * i + 2] = x.z;
-            ka[4 * i + 3] = x.w;
-          }
-          f32x4 acc = {-mref, -mref, -mref, -mref};
-#pragma unroll
-          for (int st = 0; st < 16; ++st)
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[st], qb[st], acc, 0, 0, 0);
-          s[kt4] = acc;
-        }
-        if (kbase + kKeys - 1 > min_pos || okb != 15) {
-#pragma unroll
-          for (int kt4 = 0; kt4 < 4; ++kt4)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int kp = kbase + 16 * kt4 + 4 * g + e;
-              s[kt4][e] = (kp <= rp && ((okb >> kt4) & 1)) ? s[kt4][e] : -INFINITY;
-            }
-        }
-        // Online softmax on s - mref, the reference max raised lazily (as in the
-        // 16-bit kernel: O and l rescaled only when a row's max grows past
-        // m + kLazyMax somewhere in the wave).
-        float mx = -INFINITY;
-#pragma unroll
-        for (int kt4 = 0; kt4 < 4; ++kt4)
-          mx = fmaxf(mx, fmaxf(fmaxf(s[kt4][0], s[kt4][1]), fmaxf(s[kt4][2], s[kt4][3])));
-        mx = group_max4(mx);
-        const bool grow = m == -INFINITY ? mx != -INFINITY : mx > kLazyMax;
-        if (__builtin_amdgcn_ballot_w64(grow) != 0) {
-          const float m_new = fmaxf(m, mref + mx);
-          const float corr = m_new == -INFINITY ? 1.0f : exp2_weight(m - m_new);  // m = -inf: 0
-          l *= corr;
-#pragma unroll
-          for (int mt = 0; mt < 4; ++mt) o[mt] *= corr;
-          m = m_new;
-          const float shift = (m_new == -INFINITY ? 0.0f : m_new) - mref;
-#pragma unroll
-          for (int kt4 = 0; kt4 < 4; ++kt4) s[kt4] -= shift;
-        }
-        float sum = 0.0f;
-#pragma unroll
-        for (int kt4 = 0; kt4 < 4; ++kt4)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            s[kt4][e] = exp2_weight(s[kt4][e]);
-            sum += s[kt4][e];
-          }
-        l += sum;
-        // O^T += V^T P^T: step (kt4, e) takes key 16 kt4 + 4g + e; lane (g, r)
-        // reads that key's V piece r (dims 4r .. 4r+3, the 4 tiles' A values).
-#pragma unroll
-        for (int kt4 = 0; kt4 < 4; ++kt4)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float4 v =
-                *reinterpret_cast<const float4*>(vt + (16 * kt4 + 4 * g + e) * 256 + 16 * r);
-            const float pw = s[kt4][e];
-            o[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.x, pw, o[0], 0, 0, 0);
-            o[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.y, pw, o[1], 0, 0, 0);
-            o[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.z, pw, o[2], 0, 0, 0);
-            o[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.w, pw, o[3], 0, 0, 0);
-          }
-        wait_tiles(max(0, min(kRingF32 - 2, seg_end - kb - 2)));
-        __syncthreads();
-      }
+      l[b] += sum;
     }
-
-    l = group_sum4(l);
-    if (row_ok) {
-      const float il = 1.0f / l;
-      float* dst = out + (size_t(t) * n_heads + h0) * 64 + 16 * g;
+    bf16x8 wp[NB][3];  // the weights in three parts: B, keys 16 kt + 4g + e
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const f32x4 v = {o[0][e], o[1][e], o[2][e], o[3][e]};
-        *reinterpret_cast<f32x4*>(dst + 4 * e) = v * il;
-      }
+    for (int b = 0; b < NB; ++b)
+      split3(make_float4(s[b][0][0], s[b][0][1], s[b][0][2], s[b][0][3]),
+             make_float4(s[b][1][0], s[b][1][1], s[b][1][2], s[b][1][3]), wp[b][0], wp[b][1],
+             wp[b][2]);
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+      auto dim = [&](const float4 x) { return mt == 0 ? x.x : mt == 1 ? x.y : mt == 2 ? x.z : x.w; };
+      bf16x8 vp[3];
+      split3(make_float4(dim(v[0][0]), dim(v[0][1]), dim(v[0][2]), dim(v[0][3])),
+             make_float4(dim(v[1][0]), dim(v[1][1]), dim(v[1][2]), dim(v[1][3])), vp[0], vp[1], vp[2]);
+#pragma unroll
+      for (int p = 0; p < 6; ++p)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+          o[b][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[kPartA[p]], wp[b][kPartB[p]],
+                                                             o[b][mt], 0, 0, 0);
     }
+    id0 = next0;
+    id1 = next1;
+  }
+
+  // The waves' (o, m, l) through LDS (the stages are idle: no DMA is left in flight), wave w
+  // finishing the quarter t = w of the dims: row r's dims 16g + 4w .. +3.
+  __syncthreads();
+  float* const xo = reinterpret_cast<float*>(smem);            // [wave][b][t][lane] float4
+  float2* const xml = reinterpret_cast<float2*>(smem + kTeams * NB * 4096);  // [wave][b][lane]
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      reinterpret_cast<f32x4*>(xo)[((wave * NB + b) * 4 + t) * 64 + lane] =
+          f32x4{o[b][0][t], o[b][1][t], o[b][2][t], o[b][3][t]};
+    xml[(wave * NB + b) * 64 + lane] = make_float2(m[b], group_sum4(l[b]));
+  }
+  __syncthreads();
+  if (wave >= 4) return;
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    float2 ml[kTeams];
+    float top = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < kTeams; ++w) {
+      ml[w] = xml[(w * NB + b) * 64 + lane];
+      top = fmaxf(top, ml[w].x);
+    }
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+    float total = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kTeams; ++w) {
+      const float c = ml[w].x == -INFINITY ? 0.0f : exp2_weight(ml[w].x - top);
+      total += ml[w].y * c;
+      sum += reinterpret_cast<const f32x4*>(xo)[((w * NB + b) * 4 + wave) * 64 + lane] * c;
+    }
+    const int t = t0 + 16 * b + r;
+    if (t < T)
+      *reinterpret_cast<f32x4*>(out + (size_t(t) * n_heads + head) * 64 + 16 * g + 4 * wave) =
+          sum * (1.0f / total);
   }
 }
 
-template <int W>
-int launch_prefill_f32(const dim3 grid, float* out, const float* q, const float* kp,
-                       const float* vp, int T, const int32_t* row_pos, const int32_t* row_seq,
-                       const ie_kv_layout& kv, int n_heads, int n_kv_heads, int n_blocks,
-                       hipStream_t stream) {
-  constexpr int lds = kRingF32 * kBufF32 + 16 * kSegTiles;  // 96 KB ring + the segment's page ids
-  static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(prefill_mfma_f32_kernel<W>),
-      hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  if (int rc = check_hip(attr, "hipFuncSetAttribute(attention_prefill_mfma_f32)")) return rc;
-  hipLaunchKernelGGL((prefill_mfma_f32_kernel<W>), grid, dim3(64 * W), lds, stream, out, q, kp,
-                     vp, T, row_pos, row_seq, kv.tables, kv.max_pages, kv.num_pages, n_heads,
-                     n_kv_heads, n_blocks);
+template <int NB, int kTeams>
+int launch_prefill_f32(float* out, const float* q, const float* kp, const float* vp, int T,
+                       const int32_t* row_pos, const int32_t* row_seq, const ie_kv_layout& kv,
+                       int n_heads, int n_kv_heads, hipStream_t stream) {
+  const int n_units = (T - 1) / (16 * NB) + 1;
+  const int64_t per_head = int64_t(n_units) * (n_heads / n_kv_heads);
+  const int spread = 8 % n_kv_heads == 0 ? 8 / n_kv_heads : 1;
+  const int64_t grid = 8 % n_kv_heads == 0 ? 8 * ((per_head + spread - 1) / spread)
+                                           : per_head * n_kv_heads;
+  if (grid * 64 * kTeams > int64_t(UINT32_MAX))
+    return fail(IE_HIP_EINVAL, "attention_prefill: too many rows");
+  hipLaunchKernelGGL((prefill_mfma_f32_kernel<NB, kTeams>), dim3(unsigned(grid)),
+                     dim3(64 * kTeams), 0, stream, out, q, kp, vp, T, row_pos, row_seq, kv.tables,
+                     kv.max_pages, kv.num_pages, n_heads, n_kv_heads, n_units);
   return check_launch("attention_prefill_mfma_f32");
 }
 
@@ -975,27 +1019,23 @@ int prefill_mfma_launch(float* out, const float* q, const void* k_pool, const vo
     // cost more than the append's q traffic saves).
     if (rope.table)
       return fail(IE_HIP_EINVAL, "attention_prefill: f32 caches take q rotated by rope_and_cache");
-    const int group = n_heads / n_kv_heads;
-    const int n_blocks = (T + kRows - 1) / kRows;
-    const dim3 grid((n_blocks + 1) / 2, n_kv_heads);
     const float* kf = static_cast<const float*>(k_pool);
     const float* vf = static_cast<const float*>(v_pool);
-    switch (group) {
-#define IE_PF32_CASE(W)                                                                      \
-  case W:                                                                                    \
-    return launch_prefill_f32<W>(grid, out, q, kf, vf, T, row_pos, row_seq, kv, n_heads,     \
-                                 n_kv_heads, n_blocks, stream);
-      IE_PF32_CASE(1)
-      IE_PF32_CASE(2)
-      IE_PF32_CASE(3)
-      IE_PF32_CASE(4)
-      IE_PF32_CASE(5)
-      IE_PF32_CASE(6)
-      IE_PF32_CASE(7)
-      IE_PF32_CASE(8)
-#undef IE_PF32_CASE
-    }
-    return fail(IE_HIP_EINVAL, "attention_prefill: at most 8 query heads per KV head");
+    // Two blocks of 16 rows per workgroup halve the splitting of K and V; 8 waves halve a
+    // workgroup's chain of key tiles, 4 leave more of them resident. Measured (us; rows on
+    // cached positions): 2 blocks x 4 waves from 1.75 workgroups per compute unit on (1,333
+    // on 1,000: 73, with 8 waves 82, one block 82); 8 waves below (512 on 8,000: 113, with 4
+    // 142); one block where two leave half the units idle (130 on 4,000: 44, two 57).
+    const int64_t cus = device_compute_units();
+    const int64_t pairs = (int64_t(T) + 31) / 32 * n_heads;
+    if (4 * pairs >= 7 * cus)
+      return launch_prefill_f32<2, 4>(out, q, kf, vf, T, row_pos, row_seq, kv, n_heads, n_kv_heads,
+                                      stream);
+    if (2 * pairs > cus)
+      return launch_prefill_f32<2, 8>(out, q, kf, vf, T, row_pos, row_seq, kv, n_heads, n_kv_heads,
+                                      stream);
+    return launch_prefill_f32<1, 8>(out, q, kf, vf, T, row_pos, row_seq, kv, n_heads, n_kv_heads,
+                                    stream);
   }
   const uint16_t* kp = static_cast<const uint16_t*>(k_pool);
   const uint16_t* vp = static_cast<const uint16_t*>(v_pool);
