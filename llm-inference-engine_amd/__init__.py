@@ -1,7 +1,8 @@
 """Host-side Python mirror of the gfx950 paged KV-cache library (libie_hip.so).
 
 The library's C ABI is declared in include/ie_hip.h; this module binds it with
-ctypes and offers the reference's kernel-launcher interface
+ctypes -- and, for the calls made per layer and step, with the CPython extension
+native_calls.so -- and offers the reference's kernel-launcher interface
 (src/cuda/kernels.cuh:69-102) over torch tensors, plus the page allocator
 (src/cuda/cuda_runner.cu:191-313) as a class. torch supplies device memory
 and streams only; all compute happens in the HIP kernels. Nothing here falls
@@ -19,6 +20,7 @@ from dataclasses import dataclass
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(PKG_DIR, "libie_hip.so")
+CALLS_PATH = os.path.join(PKG_DIR, "native_calls.so")
 PAGE_SIZE = 16
 KV_F32, KV_F16, KV_BF16 = 0, 1, 2
 KV_NAMES = {"f32": KV_F32, "f16": KV_F16, "bf16": KV_BF16}
@@ -133,6 +135,28 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_calls = None
+
+
+def _native():
+    """The CPython extension's entry points (raises if it has not been built)."""
+    global _calls
+    if _calls is None:
+        import importlib.util
+
+        import torch
+        if not os.path.exists(CALLS_PATH):
+            raise FileNotFoundError(
+                f"{CALLS_PATH} is missing: build it with __graft_entry__.build()")
+        lib()
+        spec = importlib.util.spec_from_file_location("native_calls", CALLS_PATH)
+        calls = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(calls)
+        calls.set_dtypes(torch.float32, torch.float16, torch.bfloat16)
+        _calls = calls
+    return _calls
+
+
 def last_error() -> str:
     return lib().ie_hip_last_error().decode()
 
@@ -142,19 +166,19 @@ def _check(rc: int) -> None:
         raise IeHipError(rc, last_error())
 
 
-def _ptr(t) -> int | None:
-    return None if t is None else t.data_ptr()
+_raw_stream = None
 
 
 def _stream(stream=None) -> int:
-    import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
-
-
-def _dtype_code(t) -> int:
-    import torch
-    return {torch.float32: KV_F32, torch.float16: KV_F16, torch.bfloat16: KV_BF16}[t.dtype]
+    global _raw_stream
+    if stream is not None:
+        return stream.cuda_stream
+    if _raw_stream is None:
+        import torch
+        torch.cuda.current_stream()  # initialises the device
+        get, device = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
+        _raw_stream = lambda: get(device())
+    return _raw_stream()
 
 
 def layout(tables, max_pages: int, num_pages: int, kv_dtype: int) -> KvLayout:
@@ -196,12 +220,10 @@ def rope_and_cache(q, k, v, k_pool, v_pool, table, row_pos, row_seq, tables, max
                    n_heads: int, n_kv_heads: int, head_dim: int, stream=None) -> None:
     """rope_and_cache (src/cuda/kernels.cuh:72-74); q may be None (append only)."""
     T = row_pos.numel()
-    kv = layout(tables, max_pages, k_pool.numel() // (PAGE_SIZE * n_kv_heads * head_dim),
-                _dtype_code(k_pool))
-    _check(lib().ie_hip_rope_and_cache(_ptr(q), _ptr(k), _ptr(v), _ptr(k_pool), _ptr(v_pool),
-                                       _ptr(table), table.shape[0], T, _ptr(row_pos),
-                                       _ptr(row_seq), kv, n_heads, n_kv_heads, head_dim,
-                                       _stream(stream)))
+    kv = (tables, max_pages, k_pool, n_kv_heads * head_dim)
+    _check(_native().ie_hip_rope_and_cache(
+        q, k, v, k_pool, v_pool, table, table.shape[0], T, row_pos, row_seq, kv, n_heads,
+        n_kv_heads, head_dim, _stream(stream)))
 
 
 def attention_chunk_tokens(T: int, max_context: int, kv_dtype: int = KV_F16) -> int:
@@ -224,11 +246,10 @@ def attention(out, q, k_pool, v_pool, row_pos, row_seq, tables, max_pages: int, 
               stream=None) -> None:
     """Flash-decoding attention (src/cuda/kernels.cuh:84-87)."""
     T = row_pos.numel()
-    kv = layout(tables, max_pages, k_pool.numel() // (PAGE_SIZE * n_kv_heads * head_dim),
-                _dtype_code(k_pool))
-    _check(lib().ie_hip_attention(_ptr(out), _ptr(q), _ptr(k_pool), _ptr(v_pool), T, _ptr(row_pos),
-                                  _ptr(row_seq), kv, num_chunks, chunk_tokens, _ptr(workspace),
-                                  n_heads, n_kv_heads, head_dim, _stream(stream)))
+    kv = (tables, max_pages, k_pool, n_kv_heads * head_dim)
+    _check(_native().ie_hip_attention(
+        out, q, k_pool, v_pool, T, row_pos, row_seq, kv, num_chunks, chunk_tokens, workspace,
+        n_heads, n_kv_heads, head_dim, _stream(stream)))
 
 
 NOALLOC_SCRATCH_BYTES = 16 << 20  # IE_HIP_NOALLOC_SCRATCH_BYTES
@@ -239,12 +260,10 @@ def attention_noalloc(out, q, k_pool, v_pool, row_pos, row_seq, tables, max_page
                       head_dim: int, stream=None) -> None:
     """attention() with the library's fixed device scratch in place of a workspace."""
     T = row_pos.numel()
-    kv = layout(tables, max_pages, k_pool.numel() // (PAGE_SIZE * n_kv_heads * head_dim),
-                _dtype_code(k_pool))
-    _check(lib().ie_hip_attention_noalloc(_ptr(out), _ptr(q), _ptr(k_pool), _ptr(v_pool), T,
-                                          _ptr(row_pos), _ptr(row_seq), kv, num_chunks,
-                                          chunk_tokens, n_heads, n_kv_heads, head_dim,
-                                          _stream(stream)))
+    kv = (tables, max_pages, k_pool, n_kv_heads * head_dim)
+    _check(_native().ie_hip_attention_noalloc(
+        out, q, k_pool, v_pool, T, row_pos, row_seq, kv, num_chunks, chunk_tokens, n_heads,
+        n_kv_heads, head_dim, _stream(stream)))
 
 
 def attention_plan_ints(T: int, num_chunks: int, chunk_tokens: int) -> int:
@@ -275,12 +294,10 @@ def attention_planned(out, q, k_pool, v_pool, row_pos, row_seq, tables, max_page
                       n_kv_heads: int, head_dim: int, stream=None) -> None:
     """attention() with a device copy of attention_plan()'s work list."""
     T = row_pos.numel()
-    kv = layout(tables, max_pages, k_pool.numel() // (PAGE_SIZE * n_kv_heads * head_dim),
-                _dtype_code(k_pool))
-    _check(lib().ie_hip_attention_planned(_ptr(out), _ptr(q), _ptr(k_pool), _ptr(v_pool), T,
-                                          _ptr(row_pos), _ptr(row_seq), kv, num_chunks,
-                                          chunk_tokens, _ptr(workspace), _ptr(plan), plan.numel(),
-                                          n_heads, n_kv_heads, head_dim, _stream(stream)))
+    kv = (tables, max_pages, k_pool, n_kv_heads * head_dim)
+    _check(_native().ie_hip_attention_planned(
+        out, q, k_pool, v_pool, T, row_pos, row_seq, kv, num_chunks, chunk_tokens, workspace,
+        plan, plan.numel(), n_heads, n_kv_heads, head_dim, _stream(stream)))
 
 
 def rope_cache_attention_planned(out, q, k, v, k_pool, v_pool, table, row_pos, row_seq, tables,
@@ -289,12 +306,10 @@ def rope_cache_attention_planned(out, q, k, v, k_pool, v_pool, table, row_pos, r
                                  stream=None) -> None:
     """rope_cache_attention() with a device copy of attention_plan()'s work list."""
     T = row_pos.numel()
-    kv = layout(tables, max_pages, k_pool.numel() // (PAGE_SIZE * n_kv_heads * head_dim),
-                _dtype_code(k_pool))
-    _check(lib().ie_hip_rope_cache_attention_planned(
-        _ptr(out), _ptr(q), _ptr(k), _ptr(v), _ptr(k_pool), _ptr(v_pool), _ptr(table),
-        table.shape[0], T, _ptr(row_pos), _ptr(row_seq), kv, num_chunks, chunk_tokens,
-        _ptr(workspace), _ptr(plan), plan.numel(), n_heads, n_kv_heads, head_dim,
+    kv = (tables, max_pages, k_pool, n_kv_heads * head_dim)
+    _check(_native().ie_hip_rope_cache_attention_planned(
+        out, q, k, v, k_pool, v_pool, table, table.shape[0], T, row_pos, row_seq, kv, num_chunks,
+        chunk_tokens, workspace, plan, plan.numel(), n_heads, n_kv_heads, head_dim,
         _stream(stream)))
 
 
@@ -309,13 +324,10 @@ def rope_cache_attention(out, q, k, v, k_pool, v_pool, table, row_pos, row_seq, 
                          n_heads: int, n_kv_heads: int, head_dim: int, stream=None) -> None:
     """rope_and_cache + attention of one decode step in one launch (q is not modified)."""
     T = row_pos.numel()
-    kv = layout(tables, max_pages, k_pool.numel() // (PAGE_SIZE * n_kv_heads * head_dim),
-                _dtype_code(k_pool))
-    _check(lib().ie_hip_rope_cache_attention(_ptr(out), _ptr(q), _ptr(k), _ptr(v), _ptr(k_pool),
-                                             _ptr(v_pool), _ptr(table), table.shape[0], T,
-                                             _ptr(row_pos), _ptr(row_seq), kv, num_chunks,
-                                             chunk_tokens, _ptr(workspace), n_heads, n_kv_heads,
-                                             head_dim, _stream(stream)))
+    kv = (tables, max_pages, k_pool, n_kv_heads * head_dim)
+    _check(_native().ie_hip_rope_cache_attention(
+        out, q, k, v, k_pool, v_pool, table, table.shape[0], T, row_pos, row_seq, kv, num_chunks,
+        chunk_tokens, workspace, n_heads, n_kv_heads, head_dim, _stream(stream)))
 
 
 def rope_cache_attention_prefill_supported(kv_dtype: int, n_heads: int, n_kv_heads: int,
@@ -330,13 +342,10 @@ def rope_cache_attention_prefill(out, q, k, v, k_pool, v_pool, table, row_pos, r
     """rope_and_cache + attention_prefill of one prompt chunk, q rotated inside the prefill
     kernel (q is not modified)."""
     T = row_pos.numel()
-    kv = layout(tables, max_pages, k_pool.numel() // (PAGE_SIZE * n_kv_heads * head_dim),
-                _dtype_code(k_pool))
-    _check(lib().ie_hip_rope_cache_attention_prefill(_ptr(out), _ptr(q), _ptr(k), _ptr(v),
-                                                     _ptr(k_pool), _ptr(v_pool), _ptr(table),
-                                                     table.shape[0], T, _ptr(row_pos),
-                                                     _ptr(row_seq), kv, n_heads, n_kv_heads,
-                                                     head_dim, _stream(stream)))
+    kv = (tables, max_pages, k_pool, n_kv_heads * head_dim)
+    _check(_native().ie_hip_rope_cache_attention_prefill(
+        out, q, k, v, k_pool, v_pool, table, table.shape[0], T, row_pos, row_seq, kv, n_heads,
+        n_kv_heads, head_dim, _stream(stream)))
 
 
 def attention_prefill_supported(n_heads: int, n_kv_heads: int, head_dim: int) -> bool:
@@ -347,23 +356,22 @@ def attention_prefill(out, q, k_pool, v_pool, row_pos, row_seq, tables, max_page
                       n_heads: int, n_kv_heads: int, head_dim: int, stream=None) -> None:
     """Prompt attention (src/cuda/kernels.cuh:93-96)."""
     T = row_pos.numel()
-    kv = layout(tables, max_pages, k_pool.numel() // (PAGE_SIZE * n_kv_heads * head_dim),
-                _dtype_code(k_pool))
-    _check(lib().ie_hip_attention_prefill(_ptr(out), _ptr(q), _ptr(k_pool), _ptr(v_pool), T,
-                                          _ptr(row_pos), _ptr(row_seq), kv, n_heads, n_kv_heads,
-                                          head_dim, _stream(stream)))
+    kv = (tables, max_pages, k_pool, n_kv_heads * head_dim)
+    _check(_native().ie_hip_attention_prefill(
+        out, q, k_pool, v_pool, T, row_pos, row_seq, kv, n_heads, n_kv_heads, head_dim,
+        _stream(stream)))
 
 
 def gather_rows(dst, src, rows, stream=None) -> None:
     """dst[r] = src[rows[r]] (src/cuda/kernels.cuh:101-102)."""
-    _check(lib().ie_hip_gather_rows(_ptr(dst), _ptr(src), _ptr(rows), rows.numel(), src.shape[-1],
-                                    _stream(stream)))
+    _check(_native().ie_hip_gather_rows(
+        dst, src, rows, rows.numel(), src.shape[-1], _stream(stream)))
 
 
 def argmax_rows(out, logits, stream=None) -> None:
     """out[r] = first index of the maximum of logits[r] (src/cuda/kernels.cuh:106)."""
-    _check(lib().ie_hip_argmax_rows(_ptr(out), _ptr(logits), logits.shape[0], logits.shape[1],
-                                    _stream(stream)))
+    _check(_native().ie_hip_argmax_rows(
+        out, logits, logits.shape[0], logits.shape[1], _stream(stream)))
 
 
 def matrix(data, scale=None) -> Matrix:
@@ -379,56 +387,55 @@ def matrix(data, scale=None) -> Matrix:
 
 def embedding(x, ids, e: Matrix, stream=None) -> None:
     """x[t] = E[ids[t]] widened to f32 (src/cuda/kernels.cuh:48-49)."""
-    _check(lib().ie_hip_embedding(_ptr(x), _ptr(ids), e, ids.numel(), _stream(stream)))
+    _check(_native().ie_hip_embedding(x, ids, e, ids.numel(), _stream(stream)))
 
 
 def rmsnorm(y, x, weight, eps: float, stream=None) -> None:
     """y = x / rms(x) * weight per row (src/cuda/kernels.cuh:51-53)."""
     dim = weight.numel()
-    _check(lib().ie_hip_rmsnorm(_ptr(y), _ptr(x), _ptr(weight), x.numel() // dim, dim, eps,
-                                _stream(stream)))
+    _check(_native().ie_hip_rmsnorm(y, x, weight, x.numel() // dim, dim, eps, _stream(stream)))
 
 
 def matmul(y, x, w: Matrix, bias=None, accumulate: bool = False, stream=None) -> None:
     """y (+)= x . W^T * scale + bias (src/cuda/kernels.cuh:55-62)."""
-    _check(lib().ie_hip_matmul(_ptr(y), _ptr(x), w, _ptr(bias), x.numel() // w.cols,
-                               int(accumulate), _stream(stream)))
+    _check(_native().ie_hip_matmul(
+        y, x, w, bias, x.numel() // w.cols, int(accumulate), _stream(stream)))
 
 
 def qkv_proj(q, k, v, x, w_qkv: Matrix, b_qkv=None, stream=None) -> None:
     """q, k, v = x . [Wq; Wk; Wv]^T + [bq; bk; bv] in one launch."""
     q_dim, kv_dim = q.shape[-1], k.shape[-1]
-    _check(lib().ie_hip_qkv_proj(_ptr(q), _ptr(k), _ptr(v), _ptr(x), w_qkv, _ptr(b_qkv),
-                                 x.numel() // w_qkv.cols, q_dim, kv_dim, _stream(stream)))
+    _check(_native().ie_hip_qkv_proj(
+        q, k, v, x, w_qkv, b_qkv, x.numel() // w_qkv.cols, q_dim, kv_dim, _stream(stream)))
 
 
 def gate_up_silu(out, x, w_gate: Matrix, w_up: Matrix, stream=None) -> None:
     """out = silu(x . Wg^T) * (x . Wu^T) (src/cuda/kernels.cuh:64-66)."""
-    _check(lib().ie_hip_gate_up_silu(_ptr(out), _ptr(x), w_gate, w_up, x.numel() // w_gate.cols,
-                                     _stream(stream)))
+    _check(_native().ie_hip_gate_up_silu(
+        out, x, w_gate, w_up, x.numel() // w_gate.cols, _stream(stream)))
 
 
 def rmsnorm_qkv_proj(q, k, v, x, norm, eps: float, w_qkv: Matrix, b_qkv=None,
                      stream=None) -> None:
     """qkv_proj(rmsnorm(x, norm, eps)) in one launch (no reference counterpart)."""
     q_dim, kv_dim = q.shape[-1], k.shape[-1]
-    _check(lib().ie_hip_rmsnorm_qkv_proj(_ptr(q), _ptr(k), _ptr(v), _ptr(x), _ptr(norm), eps,
-                                         w_qkv, _ptr(b_qkv), x.numel() // w_qkv.cols, q_dim,
-                                         kv_dim, _stream(stream)))
+    _check(_native().ie_hip_rmsnorm_qkv_proj(
+        q, k, v, x, norm, eps, w_qkv, b_qkv, x.numel() // w_qkv.cols, q_dim, kv_dim,
+        _stream(stream)))
 
 
 def rmsnorm_gate_up_silu(out, x, norm, eps: float, w_gate: Matrix, w_up: Matrix,
                          stream=None) -> None:
     """gate_up_silu(rmsnorm(x, norm, eps)) in one launch (no reference counterpart)."""
-    _check(lib().ie_hip_rmsnorm_gate_up_silu(_ptr(out), _ptr(x), _ptr(norm), eps, w_gate, w_up,
-                                             x.numel() // w_gate.cols, _stream(stream)))
+    _check(_native().ie_hip_rmsnorm_gate_up_silu(
+        out, x, norm, eps, w_gate, w_up, x.numel() // w_gate.cols, _stream(stream)))
 
 
 def gather_kv(dst, pool, tables, max_pages: int, seq: int, length: int, kv_dim: int,
               stream=None) -> None:
     """Contiguous fp32 copy of one sequence's paged rows."""
-    kv = layout(tables, max_pages, pool.numel() // (PAGE_SIZE * kv_dim), _dtype_code(pool))
-    _check(lib().ie_hip_gather_kv(_ptr(dst), _ptr(pool), kv, seq, length, kv_dim, _stream(stream)))
+    kv = (tables, max_pages, pool, kv_dim)
+    _check(_native().ie_hip_gather_kv(dst, pool, kv, seq, length, kv_dim, _stream(stream)))
 
 
 # -------------------------------------------------------- page allocator ----

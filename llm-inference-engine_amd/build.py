@@ -7,7 +7,8 @@ Every source under csrc/ is compiled by hipcc for gfx950 only, as HIP, with
                       no packed-FP32 VALU instructions (the host pass warns that
                       it does not know the feature; that is harmless).
 Objects are compiled in parallel into _build/ and linked into
-llm-inference-engine_amd/libie_hip.so, next to this file.
+llm-inference-engine_amd/libie_hip.so, next to this file, and binding/ into the CPython
+extension native_calls.so beside it.
 """
 from __future__ import annotations
 
@@ -16,6 +17,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
@@ -71,8 +73,29 @@ def build(verbose: bool = False) -> str:
     os.replace(tmp, LIB)
     if verbose:
         print(f"built {LIB}")
+    build_binding(verbose)
     build_probe(verbose)
     return LIB
+
+
+BINDING_SRC = os.path.join(PKG, "binding", "native_calls.cpp")
+BINDING_LIB = os.path.join(PKG, "native_calls.so")
+
+
+def build_binding(verbose: bool = False) -> str:
+    """The CPython extension that calls libie_hip.so (next to it, found by rpath)."""
+    tmp = BINDING_LIB + ".tmp"
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall",
+           "-D__HIP_PLATFORM_AMD__", f"-I{INCLUDE}", "-I/opt/rocm/include",
+           f"-I{sysconfig.get_paths()['include']}", BINDING_SRC, "-o", tmp, f"-L{PKG}",
+           "-l:libie_hip.so", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"binding build failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, BINDING_LIB)
+    if verbose:
+        print(f"built {BINDING_LIB}")
+    return BINDING_LIB
 
 
 PROBE_SRC = os.path.join(PKG, "probe", "hbm_probe.hip")

@@ -132,3 +132,30 @@ def test_switches_and_trace_ranges(ie):
     L.ie_hip_range_push(None)
     L.ie_hip_range_pop()
     L.ie_hip_range_pop()
+
+
+def test_native_calls(ie):
+    """The CPython extension's argument conversions (host only: empty launches and refused
+    ones): None and tensors as pointers, the layout tuple, a Matrix, float and bool values."""
+    import torch
+    z = lambda *s, **k: torch.zeros(*s, **k)
+    idx, tab = z(0, dtype=torch.int32), z(1, dtype=torch.int32)
+    kp = z(64, 128, dtype=torch.float16)
+    stream = type("S", (), {"cuda_stream": 0})()
+    ie.rope_and_cache(None, z(0, 128), z(0, 128), kp, kp, z(4, 64), idx, idx, tab, 1, 14, 2, 64,
+                      stream=stream)
+    one = z(1, dtype=torch.int32)
+    with pytest.raises(ie.IeHipError, match="head_dim"):
+        ie.rope_and_cache(None, z(1, 6), z(1, 6), kp, kp, z(4, 3), one, one, one, 1, 2, 2, 3,
+                          stream=stream)
+    with pytest.raises(KeyError):  # not a cache type
+        ie.rope_and_cache(None, z(0, 128), z(0, 128), z(64, 128, dtype=torch.int16), kp, z(4, 64),
+                          idx, idx, tab, 1, 14, 2, 64, stream=stream)
+    w = ie.matrix(z(16, 32, dtype=torch.bfloat16))
+    ie.matmul(z(0, 16), z(0, 32), w, accumulate=True, stream=stream)
+    ie.rmsnorm(z(0, 32), z(0, 32), z(32), 1e-6, stream=stream)
+    calls = ie._native()
+    with pytest.raises(TypeError):
+        calls.ie_hip_matmul(0, 0)
+    with pytest.raises(TypeError):
+        calls.ie_hip_matmul(0, 0, b"short", None, 0, 0, 0)
