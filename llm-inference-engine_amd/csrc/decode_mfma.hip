@@ -598,10 +598,18 @@ decode_partial_mfma(float* __restrict__ out, float* __restrict__ part_o,
 //     own KV head's 64 (o[4 kv_r + e][t]).
 // K goes straight into registers; V into LDS by DMA (8 KB per page, two page
 // buffers per wave), the next page's loads in flight while the wave computes.
-// One wave per (row, chunk); the grid is numbered as for the 16-bit kernel.
+//
+// One workgroup per (row, chunk), the grid numbered as for the 16-bit kernel; its W waves
+// take the chunk's pages in turn and merge their (o, m, l) through LDS. A page is a chain of
+// 64 matrix instructions of 32 cycles and the round trip of its 16 KB, ~1 us for a wave by
+// itself, so most chunk sizes take 4 waves (48 rows of 256 to 2,048 positions in chunks of
+// 128 were 455 waves on 1,024 SIMDs: 19.5 -> 12.0 us under the profiler's trace, 21.9 -> 18.4
+// with the merge); see decode_mfma_f32 for the sizes that take one. The count follows from
+// the chunk size alone, so a row's result does not depend on the launch.
 constexpr int kPageF32 = 16 * kKvd * 4;  // bytes of one f32 page of one pool
 
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
+template <int W>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(3)))
 decode_partial_mfma_f32(float* __restrict__ out, float* __restrict__ part_o,
                         float* __restrict__ part_ml, const float* __restrict__ q,
                         const float* __restrict__ k_pool, const float* __restrict__ v_pool,
@@ -610,7 +618,8 @@ decode_partial_mfma_f32(float* __restrict__ out, float* __restrict__ part_o,
                         int n_heads, int group, int num_chunks, int chunk_tokens,
                         const int32_t* __restrict__ plan) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int wave = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, r = lane & 15;
   // Which (row, chunk) this workgroup takes and the chunk's page ids, one per
   // lane: from a host-built work list in one round trip (header, item and the
@@ -676,7 +685,8 @@ decode_partial_mfma_f32(float* __restrict__ out, float* __restrict__ part_o,
   // bytes land at base + 16 l). A page outside the pool loads page 0 and is
   // masked in the math.
   float4 kv[8];
-  const unsigned vbuf_lds = lds_address(smem);
+  unsigned char* const vbuf = smem + wave * 2 * kPageF32;
+  const unsigned vbuf_lds = lds_address(vbuf);
   auto issue = [&](const int j, const int pid) {
     __builtin_amdgcn_sched_barrier(0);
     const float4* krow =
@@ -690,8 +700,8 @@ decode_partial_mfma_f32(float* __restrict__ out, float* __restrict__ part_o,
     for (int u = 0; u < 8; ++u) dma16_nt(vsrc + u * 1024, dst + u * 1024);
     __builtin_amdgcn_sched_barrier(0);
   };
-  int cur = page_id(0), nxt = page_id(1);
-  issue(0, valid(cur) ? cur : 0);  // a located chunk has at least one position
+  int cur = page_id(wave), nxt = page_id(wave + W);
+  if (wave < npg) issue(0, valid(cur) ? cur : 0);
   float qb[32];
   {
     const float qm = mine ? 0.125f * kLog2e : 0.0f;
@@ -708,22 +718,24 @@ decode_partial_mfma_f32(float* __restrict__ out, float* __restrict__ part_o,
   f32x4 o[8];
 #pragma unroll
   for (int mt = 0; mt < 8; ++mt) o[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int j = 0; j < npg; ++j) {
-    // S^T of page j: lane (g, r) gets tokens 4g + e of head r.
-    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+  for (int j = wave, it = 0; j < npg; j += W, ++it) {
+    // S^T of page j: lane (g, r) gets tokens 4g + e of head r. Four sums side by side:
+    // a chain of 32 products on one accumulator held the wave up.
+    f32x4 s = {0.f, 0.f, 0.f, 0.f}, s1 = s, s2 = s, s3 = s;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       s = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i].x, qb[4 * i + 0], s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i].y, qb[4 * i + 1], s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i].z, qb[4 * i + 2], s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i].w, qb[4 * i + 3], s, 0, 0, 0);
+      s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i].y, qb[4 * i + 1], s1, 0, 0, 0);
+      s2 = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i].z, qb[4 * i + 2], s2, 0, 0, 0);
+      s3 = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i].w, qb[4 * i + 3], s3, 0, 0, 0);
     }
+    s = (s + s1) + (s2 + s3);
     const bool ok = valid(cur);
-    const bool more = j + 1 < npg;
-    if (more) {  // page j+1: K into `kv` (just consumed), V into the other buffer
-      issue(j + 1, valid(nxt) ? nxt : 0);
+    const bool more = j + W < npg;
+    if (more) {  // the wave's next page: K into `kv` (just consumed), V into the other buffer
+      issue(it + 1, valid(nxt) ? nxt : 0);
       cur = nxt;
-      nxt = page_id(j + 2);
+      nxt = page_id(j + 2 * W);
     }
     const int tj = 16 * j;  // first token of the page within the chunk
     const bool full = tj + 16 <= n && ok;
@@ -748,7 +760,7 @@ decode_partial_mfma_f32(float* __restrict__ out, float* __restrict__ part_o,
       wait_vmcnt<16>();
     else
       wait_vmcnt<0>();
-    const float* vt = reinterpret_cast<const float*>(smem + (j & 1) * kPageF32);
+    const float* vt = reinterpret_cast<const float*>(vbuf + (it & 1) * kPageF32);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int tok = 4 * g + e;
@@ -769,13 +781,51 @@ decode_partial_mfma_f32(float* __restrict__ out, float* __restrict__ part_o,
     }
   }
   l = group_sum4(l);
-  if (!head_ok) return;
   // Head r's dims 16g + 4e' .. +3 of its own KV head: o[4 kv_r + 0..3][e'].
+  f32x4 od[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    od[e] = kv_r ? f32x4{o[4][e], o[5][e], o[6][e], o[7][e]} : f32x4{o[0][e], o[1][e], o[2][e], o[3][e]};
+  if constexpr (W > 1) {
+    // The waves' results through their V buffers (idle: every load was waited for and read),
+    // merged in wave order; wave w finishes the parts e' = w, w + W, ..
+    f32x4* const xo = reinterpret_cast<f32x4*>(vbuf);             // [e'][lane]
+    float2* const xml = reinterpret_cast<float2*>(vbuf + 4096);   // [lane]
+#pragma unroll
+    for (int e = 0; e < 4; ++e) xo[e * 64 + lane] = od[e];
+    xml[lane] = make_float2(m, l);
+    __syncthreads();
+    float mw[W], cw[W];
+    m = -INFINITY;
+    l = 0.0f;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const float2 x = reinterpret_cast<const float2*>(smem + w * 2 * kPageF32 + 4096)[lane];
+      mw[w] = x.x;
+      cw[w] = x.y;
+      m = fmaxf(m, x.x);
+    }
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const float c = mw[w] == -INFINITY ? 0.0f : exp2_weight(mw[w] - m);
+      l = __builtin_fmaf(cw[w], c, l);
+      cw[w] = c;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      od[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (e % W != wave) continue;
+#pragma unroll
+      for (int w = 0; w < W; ++w)
+        od[e] += reinterpret_cast<const f32x4*>(smem + w * 2 * kPageF32)[e * 64 + lane] * cw[w];
+    }
+  }
+  if (!head_ok) return;
   const size_t head = size_t(t) * n_heads + r;
-  const int b = 4 * kv_r;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const f32x4 v = {o[b][e], o[b + 1][e], o[b + 2][e], o[b + 3][e]};
+    if (W > 1 && e % W != wave) continue;
+    const f32x4 v = od[e];
     const int d = 16 * g + 4 * e;
     if (single) {
       *reinterpret_cast<f32x4*>(out + head * 64 + d) = v * (1.0f / l);
@@ -784,7 +834,7 @@ decode_partial_mfma_f32(float* __restrict__ out, float* __restrict__ part_o,
       *reinterpret_cast<f32x4*>(part_o + slot * 64 + d) = v;
     }
   }
-  if (!single && g == 0) {
+  if (!single && g == 0 && wave == 0) {
     const size_t slot = head * num_chunks + c;
     *reinterpret_cast<float2*>(part_ml + 2 * slot) = make_float2(m, l);
   }
@@ -893,11 +943,23 @@ int decode_mfma_f32(float* out, const float* q, const void* k_pool, const void* 
   if ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_pool) |
        reinterpret_cast<uintptr_t>(v_pool)) & 15)
     return fail(IE_HIP_EINVAL, "attention: q, out and the pools must be 16-byte aligned");
-  hipLaunchKernelGGL(decode_partial_mfma_f32, dim3(static_cast<unsigned>(slots)), dim3(64),
-                     2 * kPageF32, stream, out, ws.part_o, ws.part_ml, q,
-                     static_cast<const float*>(k_pool), static_cast<const float*>(v_pool), row_pos,
-                     row_seq, kv.tables, T, kv.max_pages, kv.num_pages, n_heads,
-                     n_heads / n_kv_heads, num_chunks, chunk_tokens, plan);
+  auto launch = [&](auto kernel, int waves) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(slots)), dim3(64 * waves),
+                       waves * 2 * kPageF32, stream, out, ws.part_o, ws.part_ml, q,
+                       static_cast<const float*>(k_pool), static_cast<const float*>(v_pool), row_pos,
+                       row_seq, kv.tables, T, kv.max_pages, kv.num_pages, n_heads,
+                       n_heads / n_kv_heads, num_chunks, chunk_tokens, plan);
+  };
+  // Waves per chunk, from its size alone (us; rows x positions, f32): 192 positions are
+  // chosen where workgroups abound (64 x 128-4,096: one wave 28.8, four 32.0), 32 hold two
+  // pages (16 x 512-2,048: 11.5 against 15.7); 64 and 128 are chosen for small grids
+  // (16 x 512-2,048 at 64: 12.4 against 12.0; 48 x 256-2,048 at 128: 19.6 against 18.4), and a
+  // chunk of more than 192 is a long chain for one wave (16 x 512-2,048 at 256: 26.6 against
+  // 15.7).
+  if (chunk_tokens <= 32 || (chunk_tokens > 128 && chunk_tokens <= 192))
+    launch(decode_partial_mfma_f32<1>, 1);
+  else
+    launch(decode_partial_mfma_f32<4>, 4);
   if (int rc = check_launch("attention_mfma_f32")) return rc;
   return decode_merge(out, ws, row_pos, T, n_heads, num_chunks, chunk_tokens, stream);
 }

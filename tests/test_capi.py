@@ -142,11 +142,12 @@ def test_native_calls(ie):
     idx, tab = z(0, dtype=torch.int32), z(1, dtype=torch.int32)
     kp = z(64, 128, dtype=torch.float16)
     stream = type("S", (), {"cuda_stream": 0})()
-    ie.rope_and_cache(None, z(0, 128), z(0, 128), kp, kp, z(4, 64), idx, idx, tab, 1, 14, 2, 64,
-                      stream=stream)
+    with pytest.raises(ie.IeHipError, match="null pointer"):  # an empty tensor has no address
+        ie.rope_and_cache(None, z(1, 128), z(1, 128), kp, kp, z(4, 64), idx, idx, tab, 1, 14, 2, 64,
+                          stream=stream)
     one = z(1, dtype=torch.int32)
     with pytest.raises(ie.IeHipError, match="head_dim"):
-        ie.rope_and_cache(None, z(1, 6), z(1, 6), kp, kp, z(4, 3), one, one, one, 1, 2, 2, 3,
+        ie.rope_and_cache(None, z(1, 64), z(1, 64), kp, kp, z(4, 32), one, one, tab, 1, 2, 2, 32,
                           stream=stream)
     with pytest.raises(KeyError):  # not a cache type
         ie.rope_and_cache(None, z(0, 128), z(0, 128), z(64, 128, dtype=torch.int16), kp, z(4, 64),

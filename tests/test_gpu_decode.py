@@ -432,3 +432,43 @@ def test_batch_shapes(ie, O, dev, case, kv):
         got = from_dev(out)
         check(O, got[live], want, kvt, f"call {call}, chunk {ct}, {ncall} chunks")
         assert np.all(got[~live] == 7.0), "rows with position -1 must be left untouched"
+
+
+@pytest.mark.parametrize("chunk_tokens", [16, 32, 48, 64, 128, 144, 192, 208, 1024])
+@pytest.mark.parametrize("planned", [False, True])
+def test_f32_waves_per_chunk(ie, O, dev, chunk_tokens, planned):
+    """f32 caches: every wave count per chunk, with chunks whose pages do not divide among the
+    waves, last chunks of one position, rows shorter than a chunk, and a page outside the
+    pool, against the oracle (the row with that page against the VALU kernel)."""
+    lens = [1, 17, chunk_tokens, chunk_tokens + 1, 2 * chunk_tokens - 15, 700]
+    rng = np.random.default_rng(chunk_tokens)
+    tables, max_pages, num_pages = make_tables(lens, rng)
+    tables[5, 3] = num_pages + 1
+    kp, vp = kv_pool(rng, num_pages, 0, O), kv_pool(rng, num_pages, 0, O)
+    pos = np.array([n - 1 for n in lens], np.int32)
+    seq = np.arange(len(lens), dtype=np.int32)
+    q = normal(rng, (len(lens), QD))
+    nc = ie.attention_chunks(max(lens), chunk_tokens)
+
+    def run():
+        ws = ie.attention_workspace(len(lens), NH, HD, nc)
+        out = torch.full((len(lens), QD), float("nan"), device=dev)
+        args = (out, to_dev(q, dev), to_dev(kp, dev, 0), to_dev(vp, dev, 0), to_dev(pos, dev),
+                to_dev(seq, dev), to_dev(tables, dev), max_pages, nc, chunk_tokens, ws)
+        if planned:
+            plan = to_dev(ie.attention_plan(pos, seq, tables, nc, chunk_tokens), dev)
+            ie.attention_planned(*args, plan, NH, NKV, HD)
+        else:
+            ie.attention(*args, NH, NKV, HD)
+        torch.cuda.synchronize()
+        return from_dev(out)
+
+    got = run()
+    want = O.paged_attention(q[:5], kp, vp, 0, pos[:5], seq[:5], tables, max_pages, NH, NKV, HD,
+                             threads=8)
+    check(O, got[:5], want, 0, f"chunk {chunk_tokens}")
+    prev = ie.set_attention_impl(ie.IMPL_VALU)
+    try:
+        check(O, got[5:], run()[5:], 0, f"chunk {chunk_tokens}, a page outside the pool")
+    finally:
+        ie.set_attention_impl(prev)
