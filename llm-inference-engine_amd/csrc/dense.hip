@@ -349,11 +349,40 @@ struct TiledLaunch {
       }
     }
   }
-  // Wide matrices (4 slots, one wave each). The 151,936-row LM head, us: at 1 to 16 tokens 64
-  // rows x 16 tokens is the best shape (1 token, bf16: 59 before, 52; INT8: 60 -> 38), from
-  // 17 on 128 x 32 (64 tokens, bf16: 138 -> 92, INT8: 177 -> 74).
+  template <int RT, int CT, int TG, bool I8>
+  bool stream_go(int per_cu, int* rc) const {
+    using Shape = StreamShape<RT, CT, TG, I8>;
+    static_assert(Shape::kLds <= kTiledMaxLds, "a compute unit's LDS");
+    const auto kernel = matmul_stream_kernel<RT, CT, TG, I8>;
+    if (Shape::kLds > 64 * 1024) {
+      static const hipError_t attr =
+          hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, Shape::kLds);
+      if ((*rc = check_hip(attr, "hipFuncSetAttribute(matmul)"))) return true;
+    }
+    const int row_tiles = (w->rows - 1) / (16 * RT) + 1;
+    const int grid = std::min(row_tiles, per_cu * device_compute_units());
+    hipLaunchKernelGGL(kernel, dim3(unsigned(grid)), dim3(64 * Shape::kWaves), unsigned(Shape::kLds),
+                       stream, y, x, w->data, w->scale, bias, T, w->rows, w->cols, accumulate, split,
+                       vec, row_tiles);
+    *rc = IE_HIP_OK;
+    return true;
+  }
+  // Wide matrices (4 slots, one wave each). Up to 64 tokens with K up to 1,024 (8 blocks a
+  // slot, held in registers) the weights are streamed past the tokens, except for 17 to 32
+  // tokens, where 128 x 32 tiles take as long and spill nothing. The 151,936-row LM head, us,
+  // direct loads before / tiles / streamed: bf16, 1 token 59 / 52 / 49, 16 tokens 74 / 64 /
+  // 57, 32 tokens 90 / 65 / 63, 64 tokens 138 / 92 / 76; INT8, 1 token 58 / 36 / 34, 16 tokens
+  // 65 / 43 / 39, 64 tokens 177 / 73 / 64. (HBM's share, at the 5.1 TB/s of a large copy:
+  // bf16 53 to 61, INT8 27 to 34.)
   bool run_wide(bool gate, int* rc) const {
     if (gate) return with_types<true, 8, 2, 4, 4, 1>(rc);
+    if (w->cols <= 32 * 4 * 8) {
+      if (T <= 16)
+        return w->int8 ? stream_go<4, 1, 1, true>(2, rc) : stream_go<2, 1, 1, false>(1, rc);
+      if (T > 32 && T <= 64)
+        return w->int8 ? stream_go<2, 2, 2, true>(1, rc) : stream_go<2, 2, 2, false>(1, rc);
+    }
     return T <= 16 ? with_types<false, 4, 1, 4, 4, 2>(rc) : with_types<false, 8, 2, 4, 4, 1>(rc);
   }
 };

@@ -117,6 +117,57 @@ __device__ __forceinline__ void tile_of_block(int b, int row_tiles, int tok_tile
   row = group * kGroup + in - tok * width;
 }
 
+// One lane's 4 rows of a finished tile: token `tok`, rows row .. row + 3.
+// vec: the row counts of every output are multiples of 4 and all pointers 16-byte
+// aligned, so they are one 16-byte access.
+template <bool GATE, bool I8, bool NORM>
+__device__ __forceinline__ void put_rows(const f32x4 (&v)[GATE ? 2 : 1], float inv, int tok, int row,
+                                         float* y, const float* scale, const float* scale2,
+                                         const float* bias, int T, int rows, int accumulate,
+                                         const RowSplit& out, int vec) {
+  constexpr int NA = GATE ? 2 : 1;
+  if (tok >= T || row >= rows) return;
+  auto place = [&](int at) {
+    if (at < out.split0) return y + size_t(tok) * out.split0 + at;
+    if (at < out.split1) return out.y1 + size_t(tok) * (out.split1 - out.split0) + (at - out.split0);
+    return out.y2 + size_t(tok) * (rows - out.split1) + (at - out.split1);
+  };
+  if (vec) {
+    f32x4 o = v[0];
+    if constexpr (I8) o *= *reinterpret_cast<const f32x4*>(scale + row);
+    if constexpr (NORM) o *= inv;
+    f32x4* dst = reinterpret_cast<f32x4*>(place(row));
+    if constexpr (GATE) {
+      f32x4 up = v[NA - 1];
+      if constexpr (I8) up *= *reinterpret_cast<const f32x4*>(scale2 + row);
+      if constexpr (NORM) up *= inv;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = silu(o[e]) * up[e];
+    } else {
+      if (bias) o += *reinterpret_cast<const f32x4*>(bias + row);
+      if (accumulate) o += *dst;
+    }
+    *dst = o;
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (row + e >= rows) break;
+    float o = v[0][e] * (I8 ? scale[row + e] : 1.0f);
+    if constexpr (NORM) o *= inv;
+    float* dst = place(row + e);
+    if constexpr (GATE) {
+      float up = v[NA - 1][e] * (I8 ? scale2[row + e] : 1.0f);
+      if constexpr (NORM) up *= inv;
+      o = silu(o) * up;
+    } else {
+      if (bias) o += bias[row + e];
+      if (accumulate) o += *dst;
+    }
+    *dst = o;
+  }
+}
+
 // GATE: out = silu(x . Wg^T * sg) * (x . Wu^T * su) (gate_up_silu); otherwise
 // y (+)= x . W^T * s + bias.
 //
@@ -163,29 +214,31 @@ matmul_tiled_kernel(float* __restrict__ y, const float* __restrict__ x, const vo
   unsigned char* const stages = tiles + wave * S * Shape::kStage;
   const unsigned stages_lds = lds_address(stages);
 
-  // DMA sources. Weight tiles: bf16, load u is row tile u, lane l row l/4, 16-byte piece
-  // (l%4) ^ (row/2 % 4); int8, load u is row tiles 2u and 2u + 1, lane l row l/2 of the 32,
-  // piece (l%2) ^ (row/4 % 2). Activations: load p is tokens 8p .. 8p+7, lane l token l/8,
-  // piece (l%8) ^ (l/8). LDS slot = lane.
-  const char* wsrc[kLA];
+  // DMA sources: a lane's byte offsets from the tile's first row and token. Weight tiles:
+  // bf16, load u is row tile u, lane l row l/4, 16-byte piece (l%4) ^ (row/2 % 4); int8,
+  // load u is row tiles 2u and 2u + 1, lane l row l/2 of the 32, piece (l%2) ^ (row/4 % 2).
+  // Activations: load p is tokens 8p .. 8p+7, lane l token l/8, piece (l%8) ^ (l/8). LDS
+  // slot = lane. (The host keeps a tile's offsets within 32 bits.)
+  constexpr int kWBytes = I8 ? 1 : 2;
+  const int wr = I8 ? lane >> 1 : lane >> 2;
+  const int wp = I8 ? (lane & 1) ^ ((wr >> 2) & 1) : (lane & 3) ^ ((wr >> 1) & 3);
+  unsigned woff[kLA];
+  bool second[kLA];  // INT8, two matrices: this lane's row tile belongs to w2
 #pragma unroll
   for (int u = 0; u < kLA; ++u) {
-    if constexpr (I8) {
-      const int wr = lane >> 1, tile = min(2 * u + (wr >> 4), NR - 1);
-      const int wp = (lane & 1) ^ ((wr >> 2) & 1);
-      wsrc[u] = static_cast<const char*>(tile / RT ? w2 : w) +
-                size_t(min(row0 + 16 * (tile % RT) + (wr & 15), rows - 1)) * cols + 16 * wp;
-    } else {
-      const int wr = lane >> 2, wp = (lane & 3) ^ ((wr >> 1) & 3);
-      wsrc[u] = static_cast<const char*>(u / RT ? w2 : w) +
-                (size_t(min(row0 + 16 * (u % RT) + wr, rows - 1)) * cols + 8 * wp) * 2;
-    }
+    const int tile = I8 ? min(2 * u + (wr >> 4), NR - 1) : u;
+    woff[u] = unsigned(min(16 * (tile % RT) + (wr & 15), rows - 1 - row0)) * unsigned(cols * kWBytes) +
+              16 * wp;
+    second[u] = tile >= RT;
   }
   const int xq = (lane & 7) ^ ((lane >> 3) & 7);
-  const float* xsrc[2 * CT];
+  unsigned xoff[2 * CT];
 #pragma unroll
   for (int p = 0; p < 2 * CT; ++p)
-    xsrc[p] = x + size_t(min(tok0 + 8 * p + (lane >> 3), T - 1)) * cols + 4 * xq;
+    xoff[p] = unsigned(min(8 * p + (lane >> 3), T - 1 - tok0)) * unsigned(cols * 4) + 16 * xq;
+  const char* const wbase = static_cast<const char*>(w) + size_t(row0) * cols * kWBytes;
+  const char* const w2base = GATE ? static_cast<const char*>(w2) + size_t(row0) * cols * kWBytes : wbase;
+  const char* const xbase = reinterpret_cast<const char*>(x + size_t(tok0) * cols);
 
   const int nblocks = cols >> 5;  // at least SLOTS (the launcher): every slot has a block
   auto blocks_of = [&](int slot) { return (nblocks - slot + SLOTS - 1) / SLOTS; };
@@ -200,15 +253,20 @@ matmul_tiled_kernel(float* __restrict__ y, const float* __restrict__ x, const vo
     const unsigned base = stages_lds + stage * Shape::kStage;
 #pragma unroll
     for (int u = 0; u < kLA; ++u) {
-      const char* src = wsrc[u] + size_t(kb) * (I8 ? 1 : 2);
+      // One matrix per load, except where a pair of INT8 row tiles straddles the two.
+      constexpr bool kPairs = I8 && GATE && RT % 2 == 1;
       if constexpr (I8 && NR % 2 == 1) {
-        if (2 * u + (lane >> 5) < NR) dma16(src, base + u * 1024);
+        if (2 * u + (lane >> 5) < NR) dma16_at(wbase + kb * kWBytes, woff[u], base + u * 1024);
+      } else if (kPairs && 2 * u + 1 == RT) {
+        dma16((second[u] ? w2base : wbase) + kb * kWBytes + woff[u], base + u * 1024);
       } else {
-        dma16(src, base + u * 1024);
+        const bool two = GATE && (I8 ? 2 * u : u) >= RT;
+        dma16_at((two ? w2base : wbase) + kb * kWBytes, woff[u], base + u * 1024);
       }
     }
 #pragma unroll
-    for (int p = 0; p < 2 * CT; ++p) dma16(xsrc[p] + kb, base + Shape::kABytes + p * 1024);
+    for (int p = 0; p < 2 * CT; ++p)
+      dma16_at(xbase + kb * 4, xoff[p], base + Shape::kABytes + p * 1024);
   };
 #pragma unroll
   for (int s = 0; s < S; ++s)
@@ -352,51 +410,138 @@ matmul_tiled_kernel(float* __restrict__ y, const float* __restrict__ x, const vo
       const float sum = total([&](int k) { return red_ss[(k * CT + j) * 64 + lane]; });
       inv = 1.0f / sqrtf(sum / float(cols) + norm.eps);
     }
-    const int tok = tok0 + 16 * j + r, row = row0 + 16 * i + 4 * g;
-    if (tok >= T || row >= rows) continue;
-    auto place = [&](int at) {
-      if (at < out.split0) return y + size_t(tok) * out.split0 + at;
-      if (at < out.split1)
-        return out.y1 + size_t(tok) * (out.split1 - out.split0) + (at - out.split0);
-      return out.y2 + size_t(tok) * (rows - out.split1) + (at - out.split1);
-    };
-    // vec: the row counts of every output are multiples of 4 and all pointers 16-byte
-    // aligned, so a lane's 4 rows are one 16-byte access.
-    if (vec) {
-      f32x4 o = v[0];
-      if constexpr (I8) o *= *reinterpret_cast<const f32x4*>(scale + row);
-      if constexpr (NORM) o *= inv;
-      f32x4* dst = reinterpret_cast<f32x4*>(place(row));
-      if constexpr (GATE) {
-        f32x4 up = v[NA - 1];
-        if constexpr (I8) up *= *reinterpret_cast<const f32x4*>(scale2 + row);
-        if constexpr (NORM) up *= inv;
+    put_rows<GATE, I8, NORM>(v, inv, tok0 + 16 * j + r, row0 + 16 * i + 4 * g, y, scale, scale2,
+                             bias, T, rows, accumulate, out, vec);
+  }
+}
+
+// The same product for a wide matrix and few tokens (the LM head of a decode step), where the
+// time is the weights' way from HBM: a persistent workgroup keeps its tokens' split
+// activations in registers and streams row tiles past them, so that nothing but weights is
+// loaded and nothing split again per tile. 4 slots x TG waves; wave (slot, tg) holds the
+// slot's at most KB K blocks of CT token tiles (12 registers a block and tile) and runs through
+// tiles of RT x 16 rows, its weights arriving in a ring of D blocks. The slots' sums meet
+// in LDS, in two buffers in turn: one barrier a tile. The order of every sum is
+// matmul_tiled_kernel's.
+template <int RT, int CT, int TG, bool I8>
+struct StreamShape {
+  static constexpr int kSlots = 4, kKB = 8, kD = 4;
+  static constexpr int kWaves = kSlots * TG;
+  static constexpr int kStage = RT * (I8 ? 512 : 1024);
+  static constexpr int kTiles = RT * CT;
+  static constexpr int kRing = kWaves * kD * kStage;
+  static constexpr int kLds = kRing + 2 * kWaves * kTiles * 1024;
+};
+
+template <int RT, int CT, int TG, bool I8>
+__global__ void __launch_bounds__(256 * TG)
+matmul_stream_kernel(float* __restrict__ y, const float* __restrict__ x, const void* __restrict__ w,
+                     const float* __restrict__ scale, const float* __restrict__ bias, int T,
+                     int rows, int cols, int accumulate, RowSplit out, int vec, int row_tiles) {
+  using Shape = StreamShape<RT, CT, TG, I8>;
+  constexpr int kSlots = Shape::kSlots, KB = Shape::kKB, D = Shape::kD;
+  constexpr int kPer = I8 ? RT / 2 : RT;  // 1 KB loads of a block
+  static_assert(!I8 || RT % 2 == 0, "INT8 loads take row tiles in pairs");
+  extern __shared__ __align__(16) unsigned char dyn[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int slot = wave / TG, tg = wave % TG;
+  const int g = lane >> 4, r = lane & 15;
+  unsigned char* const ring = dyn + wave * D * Shape::kStage;
+  const unsigned ring_lds = lds_address(ring);
+  const int nb = ((cols >> 5) - slot + kSlots - 1) / kSlots;  // this slot's blocks, 1 .. KB
+
+  // Weights: as in matmul_tiled_kernel. A tile's steps are always KB; those past the
+  // slot's blocks load 16 bytes, so that every step counts the same loads.
+  constexpr int kWBytes = I8 ? 1 : 2;
+  const int wr = I8 ? lane >> 1 : lane >> 2;
+  const int wp = I8 ? (lane & 1) ^ ((wr >> 2) & 1) : (lane & 3) ^ ((wr >> 1) & 3);
+  auto issue = [&](int tile, int b) {
+    const int kb = 32 * (slot + kSlots * min(b, nb - 1));
+    const int row0 = tile * 16 * RT;
+    const char* base = static_cast<const char*>(w) + (size_t(row0) * cols + kb) * kWBytes;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = silu(o[e]) * up[e];
-      } else {
-        if (bias) o += *reinterpret_cast<const f32x4*>(bias + row);
-        if (accumulate) o += *dst;
-      }
-      *dst = o;
-    } else {
+    for (int u = 0; u < kPer; ++u) {
+      const unsigned off = unsigned(min((I8 ? 32 : 16) * u + wr, rows - 1 - row0)) *
+                               unsigned(cols * kWBytes) + 16 * wp;
+      if (b < nb || lane == 0) dma16_at(base, off, ring_lds + (b % D) * Shape::kStage + u * 1024);
+    }
+  };
+  int tile = blockIdx.x;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (row + e >= rows) break;
-        float o = v[0][e] * (I8 ? scale[row + e] : 1.0f);
-        if constexpr (NORM) o *= inv;
-        float* dst = place(row + e);
-        if constexpr (GATE) {
-          float up = v[NA - 1][e] * (I8 ? scale2[row + e] : 1.0f);
-          if constexpr (NORM) up *= inv;
-          o = silu(o) * up;
-        } else {
-          if (bias) o += bias[row + e];
-          if (accumulate) o += *dst;
-        }
-        *dst = o;
-      }
+  for (int b = 0; b < D; ++b) issue(tile, b);
+
+  bf16x8 xb[KB][CT][3];
+#pragma unroll
+  for (int b = 0; b < KB; ++b) {
+    const int kb = 32 * (slot + kSlots * min(b, nb - 1)) + 8 * g;
+#pragma unroll
+    for (int j = 0; j < CT; ++j) {
+      const float4* src = reinterpret_cast<const float4*>(
+          x + size_t(min((tg * CT + j) * 16 + r, T - 1)) * cols + kb);
+      split3(src[0], src[1], xb[b][j][0], xb[b][j][1], xb[b][j][2]);
     }
   }
+  const int aoff = I8 ? 16 * (2 * r + ((g >> 1) ^ ((r >> 2) & 1))) + 8 * (g & 1)
+                      : 16 * (4 * r + (g ^ ((r >> 1) & 3)));
+  f32x4* const red = reinterpret_cast<f32x4*>(dyn + Shape::kRing);  // [2][wave][tile][lane]
+  for (int turn = 0; tile < row_tiles; turn ^= 1) {
+    const int next = tile + int(gridDim.x);
+    f32x4 acc[RT][CT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int j = 0; j < CT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int b = 0; b < KB; ++b) {
+      wait_vmcnt<(D - 1) * kPer>();  // this step's tile has landed
+      const unsigned char* st = ring + (b % D) * Shape::kStage;
+      bf16x8 a[RT];
+      uint2 a8[RT];
+#pragma unroll
+      for (int i = 0; i < RT; ++i) {
+        if constexpr (I8)
+          a8[i] = *reinterpret_cast<const uint2*>(st + i * 512 + aoff);
+        else
+          a[i] = *reinterpret_cast<const bf16x8*>(st + i * 1024 + aoff);
+      }
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the stage's reads are done
+      // The step D ahead; past the last tile, that tile again (read by no one).
+      if (b + D < KB)
+        issue(tile, b + D);
+      else
+        issue(next < row_tiles ? next : tile, b + D - KB);
+      if (b < nb) {
+        if constexpr (I8) {
+#pragma unroll
+          for (int i = 0; i < RT; ++i) a[i] = widen_i8(a8[i]);
+        }
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+#pragma unroll
+          for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int j = 0; j < CT; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], xb[b][j][p], acc[i][j], 0, 0, 0);
+      }
+    }
+    f32x4* const part = red + turn * Shape::kWaves * Shape::kTiles * 64;
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int j = 0; j < CT; ++j) part[(wave * Shape::kTiles + i * CT + j) * 64 + lane] = acc[i][j];
+    __syncthreads();
+    for (int u = wave; u < TG * Shape::kTiles; u += Shape::kWaves) {
+      const int t = u / Shape::kTiles, ij = u % Shape::kTiles;
+      auto of = [&](int sl) { return part[((sl * TG + t) * Shape::kTiles + ij) * 64 + lane]; };
+      const f32x4 v[1] = {(of(0) + of(2)) + (of(1) + of(3))};
+      put_rows<false, I8, false>(v, 1.0f, (t * CT + ij % CT) * 16 + r,
+                                 tile * 16 * RT + 16 * (ij / CT) + 4 * g, y, scale, nullptr, bias, T,
+                                 rows, accumulate, out, vec);
+    }
+    tile = next;
+  }
+  wait_vmcnt<0>();  // no load may land in LDS that is another workgroup's by then
 }
 
 }  // namespace iehip

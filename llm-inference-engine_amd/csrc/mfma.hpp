@@ -67,6 +67,15 @@ __device__ __forceinline__ void dma16(const void* src, unsigned lds) {
                : "memory", "m0");
 }
 
+// dma16 from a uniform base plus a lane's own byte offset: the address stays in scalar
+// registers and one 32-bit register, with no 64-bit lane arithmetic per load.
+__device__ __forceinline__ void dma16_at(const void* base, unsigned offset, unsigned lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :
+               : "v"(offset), "s"(base), "s"(lds)
+               : "memory", "m0");
+}
+
 // Loads of data read once per launch (the decode kernels' K/V pages), with the
 // non-temporal hint. A page walk of config 3's pattern (72 MB of 4 KB pages,
 // probe): plain 16-byte loads 16.8 us, non-temporal 15.6; LDS DMA 16.1,

@@ -289,10 +289,12 @@ def test_dense_argument_errors(ie, dev):
 
 
 # T, rows, cols: every LDS tile shape with ragged edges (rows % 16, rows % 4, T % 16 and the K
-# blocks' share per slot all uneven), the smallest K that takes LDS tiles and the one below it.
+# blocks' share per slot all uneven), the smallest K that takes LDS tiles and the one below it,
+# and wide matrices streamed past 16 and 64 tokens, up to the K and tokens where that ends.
 TILED = [(1, 898, 288), (17, 898, 288), (77, 898, 288), (200, 898, 288), (333, 898, 288),
          (600, 898, 288), (1003, 898, 288), (450, 1152, 896), (50, 900, 256), (50, 900, 224),
-         (9, 70001, 128), (21, 70001, 160)]
+         (9, 70001, 128), (21, 70001, 160), (16, 70001, 992), (17, 65537, 1024), (33, 70001, 224),
+         (64, 65540, 1024), (40, 66000, 1056), (65, 66000, 896)]
 
 
 @pytest.mark.parametrize("T,rows,cols", TILED)
