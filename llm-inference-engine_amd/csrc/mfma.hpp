@@ -117,6 +117,8 @@ __device__ __forceinline__ void lane_pair16(float x, float& a, float& b) {
 // possible signalling NaN in each operand (a v_max_f32 x, x, x apiece), which
 // in the softmax loops costs as many instructions as the maxima themselves.
 // For non-NaN operands both give the same value.
+// Written as inline assembly, whose operands the compiler does not space from the matrix
+// instruction that produced them: put settle() between the two.
 __device__ __forceinline__ float max_nn(float a, float b) {
   float r;
   asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
@@ -127,6 +129,19 @@ __device__ __forceinline__ float max3_nn(float a, float b, float c) {
   asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
   return r;
 }
+// The wait states (at most 11 for the instructions used here) between a matrix instruction
+// and inline assembly that reads its result, or that is given a register of a result
+// nothing reads: a VALU instruction inside assembly would read the registers as they were
+// before, or have what it wrote replaced by the result that arrives after it.
+template <int N>
+__device__ __forceinline__ void settle(f32x4 (&x)[N]) {
+  static_assert(N >= 1 && N <= 4, "accumulators of one wave tile");
+  if constexpr (N == 1) asm volatile("s_nop 11" : "+v"(x[0]));
+  if constexpr (N == 2) asm volatile("s_nop 11" : "+v"(x[0]), "+v"(x[1]));
+  if constexpr (N == 3) asm volatile("s_nop 11" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]));
+  if constexpr (N == 4) asm volatile("s_nop 11" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]));
+}
+
 __device__ __forceinline__ float group_max4(float x) {
   float a, b;
   lane_pair32(x, a, b);

@@ -649,41 +649,375 @@ int launch_prefill_variant(const dim3 grid, float* out, const float* q, const ui
                                                     stream);
 }
 
-template <int KV>
-int launch_prefill_mfma(float* out, const float* q, const uint16_t* kp, const uint16_t* vp, int T,
-                        const int32_t* row_pos, const int32_t* row_seq, const ie_kv_layout& kv,
-                        int n_heads, int n_kv_heads, const PrefillRope& rope, hipStream_t stream) {
-  const int group = n_heads / n_kv_heads;
-  const int waves = (group + kHeadsPerWave - 1) / kHeadsPerWave;
-  const int n_blocks = (T + kRows - 1) / kRows;
-  const dim3 grid((n_blocks + 1) / 2, n_kv_heads);
-  // Two teams splitting the key tiles when the grid alone leaves compute units
-  // without a workgroup or with one: twice the waves per CU, half the serial
-  // tile chain per wave. Larger grids already hold two workgroups per CU.
-  const bool teams2 = int64_t(grid.x) * grid.y <= device_compute_units();
-#define IE_PF_CASE(W)                                                                             \
-  case W:                                                                                         \
-    return teams2 ? launch_prefill_variant<KV, W, 2>(grid, out, q, kp, vp, T, row_pos, row_seq,   \
-                                                      kv, n_heads, n_kv_heads, n_blocks, rope,    \
-                                                      stream)                                     \
-                  : launch_prefill_variant<KV, W, 1>(grid, out, q, kp, vp, T, row_pos, row_seq,   \
-                                                      kv, n_heads, n_kv_heads, n_blocks, rope,    \
-                                                      stream);
-  switch (waves) {
-    IE_PF_CASE(1)
-    IE_PF_CASE(2)
-    IE_PF_CASE(3)
-    IE_PF_CASE(4)
-    IE_PF_CASE(5)
-    IE_PF_CASE(6)
-    IE_PF_CASE(7)
-    IE_PF_CASE(8)
-    default:
-      return fail(IE_HIP_EINVAL, "attention_prefill: at most 8 query heads per KV head");
+// The work of workgroup blockIdx.x in the kernels with a workgroup per row block and query
+// head. Workgroups go to the 8 XCDs in turn; where the KV heads divide 8, an XCD takes one KV
+// head's work only, so its L2 holds that head's K and V.
+__device__ __forceinline__ void unit_of_block(int n_kv_heads, int& kvh, int& unit) {
+  const int b = blockIdx.x;
+  if (8 % n_kv_heads == 0) {
+    kvh = (b & 7) % n_kv_heads;
+    unit = (b >> 3) * (8 / n_kv_heads) + (b & 7) / n_kv_heads;
+  } else {
+    kvh = b % n_kv_heads;
+    unit = b / n_kv_heads;
   }
-#undef IE_PF_CASE
 }
 
+// Workgroups for n_units row blocks; -1 where the launch's size would not fit 32 bits.
+inline int64_t unit_grid(int64_t n_units, int n_heads, int n_kv_heads, int threads) {
+  const int64_t per_head = n_units * (n_heads / n_kv_heads);
+  const int spread = 8 % n_kv_heads == 0 ? 8 / n_kv_heads : 1;
+  const int64_t grid = 8 % n_kv_heads == 0 ? 8 * ((per_head + spread - 1) / spread)
+                                           : per_head * n_kv_heads;
+  return grid * threads > int64_t(UINT32_MAX) ? -1 : grid;
+}
+
+// The waves' (o, m, l) through LDS (their stages are idle: no DMA is left in flight) and the
+// output: wave w < 4 finishes row r's dims 16g + 4w .. +3. l is the row's whole sum, in every
+// lane; o[b][mt][t] is dim 16g + 4t + mt.
+template <int NB, int kTeams>
+__device__ __forceinline__ void merge_teams(unsigned char* smem, float* out, const f32x4 (&o)[NB][4],
+                                            const float (&m)[NB], const float (&l)[NB], int t0,
+                                            int T, int n_heads, int head, int lane, int wave) {
+  const int g = lane >> 4, r = lane & 15;
+  __syncthreads();
+  f32x4* const xo = reinterpret_cast<f32x4*>(smem);                          // [wave][b][t][lane]
+  float2* const xml = reinterpret_cast<float2*>(smem + kTeams * NB * 4096);  // [wave][b][lane]
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      xo[((wave * NB + b) * 4 + t) * 64 + lane] = f32x4{o[b][0][t], o[b][1][t], o[b][2][t], o[b][3][t]};
+    xml[(wave * NB + b) * 64 + lane] = make_float2(m[b], l[b]);
+  }
+  __syncthreads();
+  if (wave >= 4) return;
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    float2 ml[kTeams];
+    float top = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < kTeams; ++w) {
+      ml[w] = xml[(w * NB + b) * 64 + lane];
+      top = fmaxf(top, ml[w].x);
+    }
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+    float total = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kTeams; ++w) {
+      const float c = ml[w].x == -INFINITY ? 0.0f : exp2_weight(ml[w].x - top);
+      total += ml[w].y * c;
+      sum += xo[((w * NB + b) * 4 + wave) * 64 + lane] * c;
+    }
+    const int t = t0 + 16 * b + r;
+    if (t < T)
+      *reinterpret_cast<f32x4*>(out + (size_t(t) * n_heads + head) * 64 + 16 * g + 4 * wave) =
+          sum * (1.0f / total);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// 16-bit caches again, one workgroup per (NB blocks of 16 rows, query head) instead of per
+// (pair of blocks, KV head): its waves take tiles of 16 KT keys in turn, each with its own K
+// stage, softmax state and output, merged through LDS at the end, as in the f32 kernel below.
+// No wave waits for another inside the key loop, and T / 16 / NB x heads workgroups fill the
+// chip where pairs of blocks x KV heads leave most of it idle. Every wave brings its own K and
+// V (prefill_mfma_kernel's 7 waves share theirs), so long prompts are bound by what a
+// compute unit can take in (4,000 rows: 68 us here, 54 there) and stay there; see
+// launch_prefill_mfma for the line.
+//   S^T and the softmax as in prefill_mfma_kernel (same operands, rounding and row sums).
+//   O^T[64 dims x 16 rows] += V^T . P^T: row i of tile mt is dim 4i + mt, so lane (g, r)'s
+//     A operand is dim 4r + mt of keys 4g + e of a page pair, and its 8-byte loads of V
+//     (16 lanes a whole 128-byte row) hold all four tiles' values: V comes straight from
+//     memory into registers, sent for before the scores, and is packed by 4 byte permutes a
+//     tile. Lane (g, r) ends up with row r's dims 16g + 4t + mt (o[mt][t]).
+template <int KV, int NB, int KT, int kTeams, bool kSplit>
+__global__ void __launch_bounds__(64 * kTeams)
+prefill_rows_kernel(float* __restrict__ out, const float* __restrict__ q,
+                    const uint16_t* __restrict__ k_pool, const uint16_t* __restrict__ v_pool, int T,
+                    const int32_t* __restrict__ row_pos, const int32_t* __restrict__ row_seq,
+                    const int32_t* __restrict__ tables, int max_pages, int num_pages, int n_heads,
+                    int n_kv_heads, int n_units, const float* __restrict__ rope,
+                    int rope_positions) {
+  using M = Mfma<KV>;
+  using op = typename M::op;
+  using E = typename M::elem;
+  static_assert(kSplit || std::is_same_v<E, _Float16>, "bf16 operands are split");
+  constexpr int kTileKeys = 16 * KT, kStage = kTileKeys * 128;
+  static_assert(KT % 2 == 0, "products over V take pages in pairs");
+  constexpr int kMerge = kTeams * NB * (4 * 1024 + 512);
+  __shared__ __align__(16) unsigned char smem[kTeams * kStage > kMerge ? kTeams * kStage : kMerge];
+  op ones;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ones[i] = static_cast<E>(1.0f);
+  const int group = n_heads / n_kv_heads;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, r = lane & 15;
+  int kvh, unit;
+  unit_of_block(n_kv_heads, kvh, unit);
+  if (unit >= n_units * group) return;
+  const int block = n_units - 1 - unit / group;  // longest contexts first
+  const int head = kvh * group + unit % group;
+  const int pos0 = __builtin_amdgcn_readfirstlane(row_pos[0]);
+  const int seq = __builtin_amdgcn_readfirstlane(row_seq[0]);
+  const int32_t* tab = tables + size_t(seq) * max_pages;
+  const int t0 = block * 16 * NB;
+  const int max_pos = pos0 + min(t0 + 16 * NB, T) - 1;
+  const int min_pos = pos0 + t0;
+  const int n_tiles = max_pos / kTileKeys + 1;
+
+  // Page ids of a tile, -1 past the table row or outside the pool.
+  auto page = [&](int at) {
+    const int id = at < max_pages ? tab[at] : -1;
+    return __builtin_amdgcn_readfirstlane(id >= 0 && id < num_pages ? id : -1);
+  };
+  // DMA of a tile's K rows, two loads a page: load h moves rows 8h .. 8h+7, lane l row
+  // 8h + l/8, LDS slot l % 8, holding piece slot ^ (row/2 % 8).
+  const unsigned row_bytes = unsigned(n_kv_heads) * 128;
+  const size_t page_bytes = size_t(IE_HIP_PAGE_SIZE) * row_bytes;
+  const char* const kbase_g = reinterpret_cast<const char*>(k_pool) + kvh * 128;
+  const char* const vbase_g = reinterpret_cast<const char*>(v_pool) + kvh * 128;
+  unsigned char* const stage = smem + wave * kStage;
+  const unsigned stage_lds = lds_address(stage);
+  unsigned koff[2], voff[4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int row = 8 * h + (lane >> 3);
+    koff[h] = row * row_bytes + 16 * ((lane & 7) ^ ((row >> 1) & 7));
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) voff[e] = (4 * g + e) * row_bytes + 8 * r;
+  auto issue_k = [&](const int (&id)[KT]) {
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) {
+      const char* base = kbase_g + size_t(max(id[kt], 0)) * page_bytes;
+      dma16_at(base, koff[0], stage_lds + kt * 2048);
+      dma16_at(base, koff[1], stage_lds + kt * 2048 + 1024);
+    }
+  };
+  int id[KT];
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) id[kt] = wave < n_tiles ? page(KT * wave + kt) : -1;
+  if (wave < n_tiles) issue_k(id);
+
+  // Row r's query of each block, times log2(e)/8: the B operands of S^T (dims 32 ks + 8g ..
+  // +7), rotated here when a RoPE table is given (the arithmetic of ie_hip_rope_and_cache;
+  // rows outside the table as they are).
+  op qhi[NB][2], qlo[NB][2];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const int t = t0 + 16 * b + r;
+    const bool row_ok = t < T;
+    const float4* src = reinterpret_cast<const float4*>(
+        q + (size_t(row_ok ? t : t0) * n_heads + head) * 64 + 8 * g);
+    float x[2][8];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const float4 a = src[8 * ks], c = src[8 * ks + 1];
+      const float v[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[ks][j] = row_ok ? v[j] : 0.0f;
+    }
+    const int rp = pos0 + t;
+    if (rope) {
+      const bool rot = row_ok && rp >= 0 && rp < rope_positions;
+      const float4* trow = reinterpret_cast<const float4*>(rope + size_t(rot ? rp : 0) * 64 + 8 * g);
+      const float4 c0 = trow[0], c1 = trow[1], s0 = trow[8], s1 = trow[9];
+      const float cs[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+      const float sn[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float x0 = x[0][j], x1 = x[1][j];
+        const float r0 = __builtin_fmaf(x0, cs[j], -(x1 * sn[j]));  // x0*c - x1*s
+        const float r1 = __builtin_fmaf(x1, cs[j], x0 * sn[j]);     // x1*c + x0*s
+        x[0][j] = rot ? r0 : x0;
+        x[1][j] = rot ? r1 : x1;
+      }
+    }
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        E hv, lv = static_cast<E>(0.0f);
+        if constexpr (kSplit) {
+          split16(x[ks][j] * (0.125f * kLog2e), hv, lv);
+        } else {
+          float xq = x[ks][j] * (0.125f * kLog2e);  // the float32 product, then its f16 rounding
+          asm("" : "+v"(xq));
+          hv = static_cast<E>(xq);
+        }
+        qhi[b][ks][j] = hv;
+        qlo[b][ks][j] = lv;
+      }
+  }
+
+  float m[NB], lsum[NB], nref[NB];  // nref: -(the reference max, 0 while m = -inf)
+  f32x4 o[NB][4];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    m[b] = -INFINITY;
+    lsum[b] = nref[b] = 0.0f;
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) o[b][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+
+  for (int tile = wave; tile < n_tiles; tile += kTeams) {
+    const int kbase = tile * kTileKeys;
+    const bool more = tile + kTeams < n_tiles;
+    int next[KT];
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) next[kt] = more ? page(KT * (tile + kTeams) + kt) : -1;
+    wait_vmcnt<0>();  // the tile's K rows have landed
+    op ka[KT][2];
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+        ka[kt][ks] = *reinterpret_cast<const op*>(stage + (16 * kt + r) * 128 +
+                                                  16 * ((4 * ks + g) ^ ((r >> 1) & 7)));
+    if (more) {
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the stage's reads are done
+      issue_k(next);
+    }
+    uint2 v[KT][4];  // key 16 kt + 4g + e, dims 4r .. 4r+3
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        v[kt][e] = *reinterpret_cast<const uint2*>(
+            vbase_g + size_t(max(id[kt], 0)) * page_bytes + voff[e]);
+
+    f32x4 s[NB][KT];
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        f32x4 acc = {nref[b], nref[b], nref[b], nref[b]};
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          acc = M::mma(ka[kt][ks], qhi[b][ks], acc);
+          if constexpr (kSplit) acc = M::mma(ka[kt][ks], qlo[b][ks], acc);
+        }
+        s[b][kt] = acc;
+      }
+#pragma unroll
+    for (int b = 0; b < NB; ++b) settle(s[b]);
+    int all = 0;
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) all |= id[kt];
+    if (kbase + kTileKeys - 1 > min_pos || all < 0) {
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int kp = kbase + 16 * kt + 4 * g + e;
+#pragma unroll
+          for (int b = 0; b < NB; ++b)
+            s[b][kt][e] = id[kt] >= 0 && kp <= pos0 + t0 + 16 * b + r ? s[b][kt][e] : -INFINITY;
+          if (id[kt] < 0 || kp > max_pos) v[kt][e] = make_uint2(0, 0);
+        }
+    }
+    // The softmax of prefill_mfma_kernel: lazily raised reference, row sums on the matrix
+    // cores from the rounded weights, the max taken only until every row has a reference
+    // (single-rounded f16) or on every tile (hi + lo).
+    op phi[NB][KT / 2], plo[NB][KT / 2];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      auto raise = [&]() {
+        float mx = max_nn(max_nn(s[b][0][0], s[b][0][1]), max_nn(s[b][0][2], s[b][0][3]));
+#pragma unroll
+        for (int kt = 1; kt < KT; ++kt)
+          mx = max3_nn(mx, max_nn(s[b][kt][0], s[b][kt][1]), max_nn(s[b][kt][2], s[b][kt][3]));
+        mx = group_max4(mx);
+        const bool grow = mx > (m[b] == -INFINITY ? -INFINITY : kLazyMax);
+        if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+          const float mref = -nref[b];
+          const float m_new = fmaxf(m[b], mref + mx);
+          const float corr = m_new == -INFINITY ? 1.0f : exp2_weight(m[b] - m_new);
+          lsum[b] *= corr;
+#pragma unroll
+          for (int mt = 0; mt < 4; ++mt) o[b][mt] *= corr;
+          m[b] = m_new;
+          const float ref = m_new == -INFINITY ? 0.0f : m_new;
+          const float shift = ref - mref;
+#pragma unroll
+          for (int kt = 0; kt < KT; ++kt) s[b][kt] -= shift;
+          nref[b] = -ref;
+        }
+      };
+      auto weights = [&]() {
+#pragma unroll
+        for (int kg = 0; kg < KT / 2; ++kg)
+#pragma unroll
+          for (int e = 0; e < 8; e += 2) {
+            const f32x4& sv = s[b][2 * kg + (e >> 2)];
+            const float p0 = exp2_weight(sv[e & 3]), p1 = exp2_weight(sv[(e & 3) + 1]);
+            E h0, h1, l0, l1;
+            if constexpr (kSplit) {
+              split16x2(p0, p1, h0, h1, l0, l1);
+              plo[b][kg][e] = l0;
+              plo[b][kg][e + 1] = l1;
+            } else {
+              round16x2(p0, p1, h0, h1);
+            }
+            phi[b][kg][e] = h0;
+            phi[b][kg][e + 1] = h1;
+          }
+      };
+      auto row_sum = [&]() {
+        f32x4 tl[1] = {{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int kg = 0; kg < KT / 2; ++kg) {
+          tl[0] = M::mma(ones, phi[b][kg], tl[0]);
+          if constexpr (kSplit) tl[0] = M::mma(ones, plo[b][kg], tl[0]);
+        }
+        // All four parts stay taken until the matrix core has written them: the next
+        // block's maxima would otherwise be put in the three that are not read.
+        settle(tl);
+        return tl[0][0];
+      };
+      if constexpr (kSplit) {
+        raise();
+        weights();
+        lsum[b] += row_sum();
+      } else {
+        const bool fresh = __builtin_amdgcn_ballot_w64(m[b] == -INFINITY) != 0;
+        if (fresh) raise();
+        weights();
+        float tl = row_sum();
+        if (!fresh && __builtin_amdgcn_ballot_w64(!(tl <= kSumMax)) != 0) {
+          raise();
+          weights();
+          tl = row_sum();
+        }
+        lsum[b] += tl;
+      }
+    }
+#pragma unroll
+    for (int kg = 0; kg < KT / 2; ++kg)
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt) {
+        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+        u32x4 a;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {  // keys 2j, 2j + 1 of the lane's 8
+          const uint2 k0 = v[2 * kg + (j >> 1)][2 * (j & 1)], k1 = v[2 * kg + (j >> 1)][2 * (j & 1) + 1];
+          a[j] = __builtin_amdgcn_perm(mt >> 1 ? k1.y : k1.x, mt >> 1 ? k0.y : k0.x,
+                                       mt & 1 ? 0x07060302u : 0x05040100u);
+        }
+        const op av = __builtin_bit_cast(op, a);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          o[b][mt] = M::mma(av, phi[b][kg], o[b][mt]);
+          if constexpr (kSplit) o[b][mt] = M::mma(av, plo[b][kg], o[b][mt]);
+        }
+      }
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) id[kt] = next[kt];
+  }
+  merge_teams<NB, kTeams>(smem, out, o, m, lsum, t0, T, n_heads, head, lane, wave);
+}
 
 // ---------------------------------------------------------------------------
 // float32 KV caches. Queries, keys, weights and values enter the 16-bit matrix cores in
@@ -736,17 +1070,8 @@ prefill_mfma_f32_kernel(float* __restrict__ out, const float* __restrict__ q,
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, r = lane & 15;
-  // Workgroups go to the 8 XCDs in turn. Where the KV heads divide 8, an XCD takes one KV
-  // head's work only, so its L2 holds that head's K and V.
-  const int spread = 8 % n_kv_heads == 0 ? 8 / n_kv_heads : 1;  // XCDs per KV head
   int kvh, unit;
-  if (8 % n_kv_heads == 0) {
-    kvh = (blockIdx.x & 7) % n_kv_heads;
-    unit = int(blockIdx.x >> 3) * spread + (blockIdx.x & 7) / n_kv_heads;
-  } else {
-    kvh = blockIdx.x % n_kv_heads;
-    unit = blockIdx.x / n_kv_heads;
-  }
+  unit_of_block(n_kv_heads, kvh, unit);
   if (unit >= n_units * group) return;
   const int block = n_units - 1 - unit / group;  // longest contexts first
   const int head = kvh * group + unit % group;
@@ -870,6 +1195,8 @@ prefill_mfma_f32_kernel(float* __restrict__ out, const float* __restrict__ q,
             s[b][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[kPartA[p]], qp[b][ks][kPartB[p]],
                                                                s[b][kt], 0, 0, 0);
       }
+#pragma unroll
+    for (int b = 0; b < NB; ++b) settle(s[b]);
     // Keys a row may not see, or in pages outside the pool: no weight, and V rows that
     // nothing may see zeroed (stale or non-finite memory must not reach O through 0 * x).
     if (kbase + kKeysF32 - 1 > min_pos || (id0 | id1) < 0) {
@@ -940,43 +1267,9 @@ prefill_mfma_f32_kernel(float* __restrict__ out, const float* __restrict__ q,
     id1 = next1;
   }
 
-  // The waves' (o, m, l) through LDS (the stages are idle: no DMA is left in flight), wave w
-  // finishing the quarter t = w of the dims: row r's dims 16g + 4w .. +3.
-  __syncthreads();
-  float* const xo = reinterpret_cast<float*>(smem);            // [wave][b][t][lane] float4
-  float2* const xml = reinterpret_cast<float2*>(smem + kTeams * NB * 4096);  // [wave][b][lane]
 #pragma unroll
-  for (int b = 0; b < NB; ++b) {
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-      reinterpret_cast<f32x4*>(xo)[((wave * NB + b) * 4 + t) * 64 + lane] =
-          f32x4{o[b][0][t], o[b][1][t], o[b][2][t], o[b][3][t]};
-    xml[(wave * NB + b) * 64 + lane] = make_float2(m[b], group_sum4(l[b]));
-  }
-  __syncthreads();
-  if (wave >= 4) return;
-#pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    float2 ml[kTeams];
-    float top = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < kTeams; ++w) {
-      ml[w] = xml[(w * NB + b) * 64 + lane];
-      top = fmaxf(top, ml[w].x);
-    }
-    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
-    float total = 0.0f;
-#pragma unroll
-    for (int w = 0; w < kTeams; ++w) {
-      const float c = ml[w].x == -INFINITY ? 0.0f : exp2_weight(ml[w].x - top);
-      total += ml[w].y * c;
-      sum += reinterpret_cast<const f32x4*>(xo)[((w * NB + b) * 4 + wave) * 64 + lane] * c;
-    }
-    const int t = t0 + 16 * b + r;
-    if (t < T)
-      *reinterpret_cast<f32x4*>(out + (size_t(t) * n_heads + head) * 64 + 16 * g + 4 * wave) =
-          sum * (1.0f / total);
-  }
+  for (int b = 0; b < NB; ++b) l[b] = group_sum4(l[b]);
+  merge_teams<NB, kTeams>(smem, out, o, m, l, t0, T, n_heads, head, lane, wave);
 }
 
 template <int NB, int kTeams>
@@ -984,16 +1277,89 @@ int launch_prefill_f32(float* out, const float* q, const float* kp, const float*
                        const int32_t* row_pos, const int32_t* row_seq, const ie_kv_layout& kv,
                        int n_heads, int n_kv_heads, hipStream_t stream) {
   const int n_units = (T - 1) / (16 * NB) + 1;
-  const int64_t per_head = int64_t(n_units) * (n_heads / n_kv_heads);
-  const int spread = 8 % n_kv_heads == 0 ? 8 / n_kv_heads : 1;
-  const int64_t grid = 8 % n_kv_heads == 0 ? 8 * ((per_head + spread - 1) / spread)
-                                           : per_head * n_kv_heads;
-  if (grid * 64 * kTeams > int64_t(UINT32_MAX))
-    return fail(IE_HIP_EINVAL, "attention_prefill: too many rows");
+  const int64_t grid = unit_grid(n_units, n_heads, n_kv_heads, 64 * kTeams);
+  if (grid < 0) return fail(IE_HIP_EINVAL, "attention_prefill: too many rows");
   hipLaunchKernelGGL((prefill_mfma_f32_kernel<NB, kTeams>), dim3(unsigned(grid)),
                      dim3(64 * kTeams), 0, stream, out, q, kp, vp, T, row_pos, row_seq, kv.tables,
                      kv.max_pages, kv.num_pages, n_heads, n_kv_heads, n_units);
   return check_launch("attention_prefill_mfma_f32");
+}
+
+template <int KV, int NB, int KT, int kTeams>
+int launch_prefill_rows(float* out, const float* q, const uint16_t* kp, const uint16_t* vp, int T,
+                        const int32_t* row_pos, const int32_t* row_seq, const ie_kv_layout& kv,
+                        int n_heads, int n_kv_heads, const PrefillRope& rope, hipStream_t stream) {
+  const int n_units = (T - 1) / (16 * NB) + 1;
+  const int64_t grid = unit_grid(n_units, n_heads, n_kv_heads, 64 * kTeams);
+  if (grid < 0) return fail(IE_HIP_EINVAL, "attention_prefill: too many rows");
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(unsigned(grid)), dim3(64 * kTeams), 0, stream, out, q, kp, vp, T,
+                       row_pos, row_seq, kv.tables, kv.max_pages, kv.num_pages, n_heads, n_kv_heads,
+                       n_units, rope.table, rope.positions);
+  };
+  if (KV == IE_KV_BF16 || prefill_rounding() == IE_HIP_PREFILL_SPLIT)
+    go(prefill_rows_kernel<KV, NB, KT, kTeams, true>);
+  else if constexpr (KV == IE_KV_F16)
+    go(prefill_rows_kernel<KV, NB, KT, kTeams, false>);
+  return check_launch("attention_prefill_rows");
+}
+
+template <int KV>
+int launch_prefill_mfma(float* out, const float* q, const uint16_t* kp, const uint16_t* vp, int T,
+                        const int32_t* row_pos, const int32_t* row_seq, const ie_kv_layout& kv,
+                        int n_heads, int n_kv_heads, const PrefillRope& rope, hipStream_t stream) {
+  const int group = n_heads / n_kv_heads;
+  const int waves = (group + kHeadsPerWave - 1) / kHeadsPerWave;
+  const int n_blocks = (T + kRows - 1) / kRows;
+  const dim3 grid((n_blocks + 1) / 2, n_kv_heads);
+  // Which kernel, from the workgroups each would have. A workgroup per (pair of blocks, KV
+  // head) shares every K/V tile among the group's heads, which pays where those workgroups
+  // fill two thirds of the compute units; below, workgroups per (row block, query head).
+  // Measured (us, f16 / bf16; rows on cached positions), pairs of blocks against row blocks:
+  // 4,000 on 0: 54 / 82 against 68 / 95; 2,000 on 0: 31 / 46 against 28 / 34; 2,000 on 2,000:
+  // 67 / 107 against 54 / 73; 600 on 0: 18 / 23 against 11 / 12; 130 on 4,000: 81 / 135 against
+  // 17 / 19. Of the row-block shapes: one block and 8 waves while that gives at most a
+  // workgroup per unit (64 on 2,000, f16: 11.1, two blocks 13); two blocks, 32-key tiles and 8
+  // waves up to 2.5 (512 on 8,000, f16: 37, 4 waves 53); 64-key tiles and 4 waves above
+  // (2,000 on 2,000, bf16: 73, 8 waves 77).
+  const int64_t cus = device_compute_units();
+  if (3 * int64_t(grid.x) * grid.y < 2 * cus) {
+    const int64_t singles = int64_t(n_blocks) * n_heads;
+    const int64_t pairs = (int64_t(T) + 31) / 32 * n_heads;
+    if (singles <= cus)
+      return launch_prefill_rows<KV, 1, 4, 8>(out, q, kp, vp, T, row_pos, row_seq, kv, n_heads,
+                                              n_kv_heads, rope, stream);
+    if (2 * pairs <= 5 * cus)
+      return launch_prefill_rows<KV, 2, 2, 8>(out, q, kp, vp, T, row_pos, row_seq, kv, n_heads,
+                                              n_kv_heads, rope, stream);
+    return launch_prefill_rows<KV, 2, 4, 4>(out, q, kp, vp, T, row_pos, row_seq, kv, n_heads,
+                                            n_kv_heads, rope, stream);
+  }
+  // Two teams splitting the key tiles when the grid alone leaves compute units
+  // without a workgroup or with one: twice the waves per CU, half the serial
+  // tile chain per wave. Larger grids already hold two workgroups per CU.
+  const bool teams2 = int64_t(grid.x) * grid.y <= cus;
+#define IE_PF_CASE(W)                                                                             \
+  case W:                                                                                         \
+    return teams2 ? launch_prefill_variant<KV, W, 2>(grid, out, q, kp, vp, T, row_pos, row_seq,   \
+                                                      kv, n_heads, n_kv_heads, n_blocks, rope,    \
+                                                      stream)                                     \
+                  : launch_prefill_variant<KV, W, 1>(grid, out, q, kp, vp, T, row_pos, row_seq,   \
+                                                      kv, n_heads, n_kv_heads, n_blocks, rope,    \
+                                                      stream);
+  switch (waves) {
+    IE_PF_CASE(1)
+    IE_PF_CASE(2)
+    IE_PF_CASE(3)
+    IE_PF_CASE(4)
+    IE_PF_CASE(5)
+    IE_PF_CASE(6)
+    IE_PF_CASE(7)
+    IE_PF_CASE(8)
+    default:
+      return fail(IE_HIP_EINVAL, "attention_prefill: at most 8 query heads per KV head");
+  }
+#undef IE_PF_CASE
 }
 
 }  // namespace

@@ -71,47 +71,54 @@ def test_prompts(ie, O, dev, case, kv, impl):
     check(O, dec, want, kvt, f"decode kernel on prompt case {case}")
 
 
-# Positions already cached, rows: each split of the f32 kernel's work, ragged.
-F32_SPLITS = [(0, 2), (500, 33), (77, 335), (3, 1030)]
+# Positions already cached, rows: each split of the kernels' work, ragged.
+SPLITS = [(0, 2), (500, 33), (77, 335), (3, 1030), (130, 1500)]
 
 
-@pytest.mark.parametrize("start,T", F32_SPLITS)
+@pytest.mark.parametrize("kv", list(KVS))
+@pytest.mark.parametrize("start,T", SPLITS)
 @pytest.mark.parametrize("hole", [False, True])
-def test_f32_work_splits(ie, O, dev, start, T, hole):
-    """Every split of the f32 prefill's rows and key tiles over workgroups and waves, with
-    NaN in every cached row that no position holds; `hole` puts one page of the sequence
-    outside the pool (its keys are skipped), checked against the sequence with those keys
-    moved out of sight."""
+def test_work_splits(ie, O, dev, kv, start, T, hole):
+    """Every split of the prefill's rows and key tiles over workgroups and waves, with NaN in
+    every cached row that no position holds; `hole` puts one page of the sequence outside
+    the pool (its keys are skipped), checked against the sequence with those keys moved out
+    of sight."""
+    kvt = KVS[kv]
     rng = np.random.default_rng(start + T)
     n = start + T
     tables, max_pages, num_pages = make_tables([n], rng, extra_pages=3)
-    kp, vp = kv_pool(rng, num_pages, 0, O), kv_pool(rng, num_pages, 0, O)
+    kp, vp = kv_pool(rng, num_pages, kvt, O), kv_pool(rng, num_pages, kvt, O)
     pos = np.arange(n)
     used = np.zeros(num_pages * 16, bool)
     used[tables[0, pos // 16] * 16 + pos % 16] = True
-    kp[~used], vp[~used] = np.nan, np.nan
+    nan = np.nan if kvt == 0 else 0x7FFF  # a NaN's bits in either 16-bit type
+    kp[~used], vp[~used] = nan, nan
     row_pos = np.arange(start, n, dtype=np.int32)
     row_seq = np.zeros(T, np.int32)
     q = normal(rng, (T, QD))
     seen = tables.copy()
     if hole and n > 48:
         seen[0, 1] = num_pages + 5  # positions 16 .. 31
-    got = gpu_prefill(ie, dev, q, kp, vp, 0, row_pos, row_seq, seen, max_pages)
+    got = gpu_prefill(ie, dev, q, kp, vp, kvt, row_pos, row_seq, seen, max_pages)
     if not hole or n <= 48:
-        want = O.paged_attention(q, kp, vp, 0, row_pos, row_seq, tables, max_pages, NH, NKV, HD,
-                                 threads=8)
-        check(O, got, want, 0, f"f32 split {start}+{T}")
+        rows = np.unique(np.linspace(0, T - 1, 40).astype(int))
+        want = O.paged_attention(q[rows], kp, vp, kvt, row_pos[rows], row_seq[rows], tables,
+                                 max_pages, NH, NKV, HD, threads=8)
+        check(O, got[rows], want, kvt, f"{kv} split {start}+{T}")
+        assert np.isfinite(got).all()
         return
+    kw, vw = (O.widen_kv(a, kvt).reshape(a.shape).astype(np.float64) if kvt else a for a in (kp, vp))
     at = tables[0, pos // 16] * 16 + pos % 16
     keep = (pos < 16) | (pos >= 32)
     for t in sorted({0, T // 2, T - 1}):
         vis = at[keep & (pos <= row_pos[t])]
         for h in range(NH):
             cols = slice(h // 7 * HD, (h // 7 + 1) * HD)
-            s = kp[vis, cols].astype(np.float64) @ q[t, h * HD:(h + 1) * HD].astype(np.float64) / 8
+            s = kw[vis, cols].astype(np.float64) @ q[t, h * HD:(h + 1) * HD].astype(np.float64) / 8
             w = np.exp(s - s.max())
-            want = (w / w.sum()) @ vp[vis, cols].astype(np.float64)
-            assert np.abs(got[t, h * HD:(h + 1) * HD] - want).max() <= 1e-5 * np.abs(want).max()
+            want = (w / w.sum()) @ vw[vis, cols].astype(np.float64)
+            bound = 2e-3 if kvt else 1e-5 * np.abs(want).max()
+            assert np.abs(got[t, h * HD:(h + 1) * HD] - want).max() <= bound
 
 
 @pytest.mark.parametrize("kv", ["f16", "bf16"])
