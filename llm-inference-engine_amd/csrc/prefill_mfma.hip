@@ -1035,7 +1035,7 @@ prefill_rows_kernel(float* __restrict__ out, const float* __restrict__ q,
 // contexts first, where a workgroup per pair of blocks and KV head left two thirds of the
 // compute units idle at 1,333 rows. What bounds it now is VALU issue: a tile's K and V take
 // 352 instructions to split, shared by NB blocks. Times (us, was 7 waves on shared f32
-// tiles): 1,333 rows on 1,000 cached 237 -> 73, 4,000 rows 281 -> 194, 130 rows on 4,000
+// tiles): 1,333 rows on 1,000 cached 237 -> 72, 4,000 rows 281 -> 193, 130 rows on 4,000
 // cached 548 -> 44.
 //   S^T[16 keys x 16 rows] per key group of 16: step ks takes dims 16g + 8ks .. +7, so lane
 //     (g, r) reads key r's dims 16g .. 16g+15 (64 bytes, 4 LDS reads).
@@ -1046,7 +1046,11 @@ prefill_rows_kernel(float* __restrict__ out, const float* __restrict__ q,
 //     scores and used after the softmax. Lane (g, r) ends up with row r's dims
 //     16g + 4t + mt (o[mt][t]).
 // K tiles (8 KB) come through LDS by DMA, one stage per wave: read whole into registers,
-// then the next tile is sent for. K rows are stored with their 16-byte pieces swizzled
+// then the next tile is sent for. Loads take a scalar page base and a 32-bit lane offset
+// (64-bit lane addresses: 1,000 rows 30.6 -> 29.5 us, 4,000 rows 198 -> 193). Four waves a
+// SIMD with one block need its registers at 128, as asked for; three with two blocks spill
+// (1,000 rows 30.6, 4,000 rows 189: not kept); three or four blocks hold so many registers
+// that too few waves are left (4,000 rows 242 and 236 us). K rows are stored with their 16-byte pieces swizzled
 // (piece ^ (key & 15)), so the 16 lanes of a group reading the same dims of 16 keys hit
 // distinct banks.
 constexpr int kKeysF32 = 32;                      // keys per wave tile (2 pages)
@@ -1057,6 +1061,7 @@ __device__ constexpr int kPartB[6] = {0, 2, 1, 0, 1, 0};
 
 template <int NB, int kTeams>
 __global__ void __launch_bounds__(64 * kTeams)
+__attribute__((amdgpu_waves_per_eu(NB == 1 ? 4 : 2)))
 prefill_mfma_f32_kernel(float* __restrict__ out, const float* __restrict__ q,
                         const float* __restrict__ k_pool, const float* __restrict__ v_pool, int T,
                         const int32_t* __restrict__ row_pos, const int32_t* __restrict__ row_seq,
@@ -1075,7 +1080,6 @@ prefill_mfma_f32_kernel(float* __restrict__ out, const float* __restrict__ q,
   if (unit >= n_units * group) return;
   const int block = n_units - 1 - unit / group;  // longest contexts first
   const int head = kvh * group + unit % group;
-  const int kv_dim = n_kv_heads * 64;
   const int pos0 = __builtin_amdgcn_readfirstlane(row_pos[0]);
   const int seq = __builtin_amdgcn_readfirstlane(row_seq[0]);
   const int32_t* tab = tables + size_t(seq) * max_pages;
@@ -1109,13 +1113,13 @@ prefill_mfma_f32_kernel(float* __restrict__ out, const float* __restrict__ q,
   };
   // DMA of a tile's K rows: load u moves keys 4u .. 4u+3, lane l key 4u + l/16, LDS slot
   // l % 16, holding piece slot ^ (key & 15).
-  const size_t row_bytes = size_t(kv_dim) * 4;
+  const unsigned row_bytes = unsigned(n_kv_heads) * 256;
   const size_t page_bytes = size_t(IE_HIP_PAGE_SIZE) * row_bytes;
   const char* const kbase_g = reinterpret_cast<const char*>(k_pool) + kvh * 256;
   const char* const vbase_g = reinterpret_cast<const char*>(v_pool) + kvh * 256;
   unsigned char* const stage = smem + wave * kStageF32;
   const unsigned stage_lds = lds_address(stage);
-  size_t koff[4], voff[4];
+  unsigned koff[4], voff[4];
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int key = 4 * u + g;
@@ -1125,8 +1129,8 @@ prefill_mfma_f32_kernel(float* __restrict__ out, const float* __restrict__ q,
   auto issue_k = [&](int ida, int idb) {
 #pragma unroll
     for (int u = 0; u < 8; ++u)
-      dma16(kbase_g + size_t(max(u < 4 ? ida : idb, 0)) * page_bytes + koff[u & 3],
-            stage_lds + u * 1024);
+      dma16_at(kbase_g + size_t(max(u < 4 ? ida : idb, 0)) * page_bytes, koff[u & 3],
+               stage_lds + u * 1024);
   };
 
   float m[NB], l[NB];  // running max (base 2), this lane's part of the sum
