@@ -674,11 +674,12 @@ inline int64_t unit_grid(int64_t n_units, int n_heads, int n_kv_heads, int threa
 
 // The waves' (o, m, l) through LDS (their stages are idle: no DMA is left in flight) and the
 // output: wave w < 4 finishes row r's dims 16g + 4w .. +3. l is the row's whole sum, in every
-// lane; o[b][mt][t] is dim 16g + 4t + mt.
-template <int NB, int kTeams>
+// lane; o[b][mt][t] is dim 16g + 4t + mt. after(b, x, dst) follows block b's result x into `out`.
+template <int NB, int kTeams, typename After>
 __device__ __forceinline__ void merge_teams(unsigned char* smem, float* out, const f32x4 (&o)[NB][4],
                                             const float (&m)[NB], const float (&l)[NB], int t0,
-                                            int T, int n_heads, int head, int lane, int wave) {
+                                            int T, int n_heads, int head, int lane, int wave,
+                                            After after) {
   const int g = lane >> 4, r = lane & 15;
   __syncthreads();
   f32x4* const xo = reinterpret_cast<f32x4*>(smem);                          // [wave][b][t][lane]
@@ -710,9 +711,11 @@ __device__ __forceinline__ void merge_teams(unsigned char* smem, float* out, con
       sum += xo[((w * NB + b) * 4 + wave) * 64 + lane] * c;
     }
     const int t = t0 + 16 * b + r;
-    if (t < T)
-      *reinterpret_cast<f32x4*>(out + (size_t(t) * n_heads + head) * 64 + 16 * g + 4 * wave) =
-          sum * (1.0f / total);
+    f32x4* const dst =
+        reinterpret_cast<f32x4*>(out + (size_t(t) * n_heads + head) * 64 + 16 * g + 4 * wave);
+    const f32x4 x = sum * (1.0f / total);
+    if (t < T) *dst = x;
+    after(b, x, dst);
   }
 }
 
@@ -1016,7 +1019,8 @@ prefill_rows_kernel(float* __restrict__ out, const float* __restrict__ q,
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) id[kt] = next[kt];
   }
-  merge_teams<NB, kTeams>(smem, out, o, m, lsum, t0, T, n_heads, head, lane, wave);
+  merge_teams<NB, kTeams>(smem, out, o, m, lsum, t0, T, n_heads, head, lane, wave,
+                          [](int, f32x4, f32x4*) {});
 }
 
 // ---------------------------------------------------------------------------
@@ -1273,7 +1277,61 @@ prefill_mfma_f32_kernel(float* __restrict__ out, const float* __restrict__ q,
 
 #pragma unroll
   for (int b = 0; b < NB; ++b) l[b] = group_sum4(l[b]);
-  merge_teams<NB, kTeams>(smem, out, o, m, l, t0, T, n_heads, head, lane, wave);
+
+  // What three bf16 parts cannot hold: infinities, NaN and what rounds to infinity in bf16 (from
+  // 3.3962e38 on) make every output that they reach NaN, their last part being one, and
+  // outputs all of whose values are below 2^-110 lack the values' low parts. A wave that
+  // has written such an output (not finite, or below 2^-100) takes block b's rows over all their
+  // keys again with the whole float32 values, on the f32 instruction, for its own 16 dims.
+  // (Looked for after the write: no size is slower by more than 2%; every wave looking at its
+  // own sums before the merge took 1.4 us more a launch.)
+  auto redo = [&](int b, f32x4 x, f32x4* dst) {
+    const int row = t0 + 16 * b + r;
+    bool odd = false;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      odd |= !(x[e] == 0.0f || (fabsf(x[e]) >= 0x1p-100f && fabsf(x[e]) < INFINITY));
+    if (__builtin_amdgcn_ballot_w64(odd && row < T) == 0) return;
+    const float* src = q + (size_t(row < T ? row : t0) * n_heads + head) * 64 + 16 * g;
+    float qv[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) qv[i] = row < T ? src[i] * (0.125f * kLog2e) : 0.0f;
+    const int last = min(pos0 + t0 + 16 * b + 15, max_pos);
+    float top = -INFINITY, total = 0.0f;  // running max, this lane's part of the sum
+    x = f32x4{0.f, 0.f, 0.f, 0.f};        // row r, dims 16g + 4 wave + e
+#pragma nounroll
+    for (int u = 0; 16 * u <= last; ++u) {
+      const int id = page(u);
+      if (id < 0) continue;
+      const size_t at = size_t(id) * page_bytes;
+      const float* krow = reinterpret_cast<const float*>(kbase_g + at + r * row_bytes) + 16 * g;
+      f32x4 sc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 16; ++i)  // step i: dim 16g + i of key r
+        sc = __builtin_amdgcn_mfma_f32_16x16x4f32(krow[i], qv[i], sc, 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (16 * u + 4 * g + e > pos0 + row) sc[e] = -INFINITY;
+      const float was = top;
+      top = fmaxf(top, group_max4(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]))));
+      if (top != -INFINITY) {
+        const float corr = exp2_weight(was - top);
+        total *= corr;
+        x *= corr;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {  // step e: key 4g + e, row r of the tile dim 16 (r/4) + r%4
+        const float w = top == -INFINITY ? 0.0f : exp2_weight(sc[e] - top);
+        total += w;
+        const float* vrow = reinterpret_cast<const float*>(vbase_g + at + (4 * g + e) * row_bytes);
+        const float v = 16 * u + 4 * g + e <= last ? vrow[16 * (r >> 2) + 4 * wave + (r & 3)] : 0.0f;
+        x = __builtin_amdgcn_mfma_f32_16x16x4f32(v, w, x, 0, 0, 0);
+      }
+    }
+    x *= 1.0f / group_sum4(total);
+    if (row < T) *dst = x;
+  };
+  merge_teams<NB, kTeams>(smem, out, o, m, l, t0, T, n_heads, head, lane, wave, redo);
 }
 
 template <int NB, int kTeams>

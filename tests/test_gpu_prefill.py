@@ -121,6 +121,71 @@ def test_work_splits(ie, O, dev, kv, start, T, hole):
             assert np.abs(got[t, h * HD:(h + 1) * HD] - want).max() <= bound
 
 
+def attend64(q, k, v, row_pos, heads_of):
+    """Causal attention in float64 of rows at `row_pos` over contiguous [n, kv dims] float64
+    keys and values; heads_of(h) gives query head h's columns of k and v."""
+    out = np.empty(q.shape)
+    for t, p in enumerate(row_pos):
+        for h in range(q.shape[1] // HD):
+            cols, hs = heads_of(h), slice(h * HD, (h + 1) * HD)
+            s = k[: p + 1, cols] @ q[t, hs].astype(np.float64) / 8
+            w = np.exp(s - s.max())
+            out[t, hs] = (w / w.sum()) @ v[: p + 1, cols]
+    return out
+
+
+@pytest.mark.parametrize("start,T", [(40, 90), (77, 500), (3, 1100)])
+@pytest.mark.parametrize("what", ["k_minus_inf", "k_huge", "k_nan", "v_inf", "v_huge", "v_tiny"])
+def test_f32_extreme_values(ie, O, dev, what, start, T):
+    """f32 caches over the whole range of float32: a key whose score is -inf takes no weight,
+    values above bf16's largest and below its precise range keep float32 accuracy, infinite
+    values come out infinite and NaN as NaN, and rows before such a position (a block of 16
+    further up) see nothing of it. Each split of the prefill's work."""
+    rng = np.random.default_rng(start + T)
+    n = start + T
+    tables, max_pages, num_pages = make_tables([n], rng)
+    at = tables[0, np.arange(n) // 16] * 16 + np.arange(n) % 16
+    k, v, q = normal(rng, (n, KVD)), normal(rng, (n, KVD)), normal(rng, (T, QD))
+    p = start + T // 64 * 32 + 21  # the position that is unlike the others
+    first = (p - start) // 16 * 16  # rows before this one must not notice it
+    if what == "k_minus_inf":
+        p, first = start - 2, 0  # a cached position: every row sees it
+        k[p, 0] = -np.inf
+        q[:, 0:QD // 2:HD] = np.abs(q[:, 0:QD // 2:HD]) + 0.5
+    elif what == "k_huge":
+        k[::7, 5], q[:, 5:QD // 2:HD] = -3.4e38, 1e-30  # scores of -4e7
+    elif what == "k_nan":
+        k[p, 70] = np.nan
+    elif what == "v_inf":
+        v[p, 3] = np.inf
+    elif what == "v_huge":
+        v[p, 3], k[p] = 3.4e38, 0
+    else:
+        v[:, 9] *= np.float32(1e-36)
+    kp, vp = (np.zeros((num_pages * 16, KVD), np.float32) for _ in range(2))
+    kp[at], vp[at] = k, v
+    row_pos = np.arange(start, n, dtype=np.int32)
+    got = gpu_prefill(ie, dev, q, kp, vp, 0, row_pos, np.zeros(T, np.int32), tables, max_pages)
+    rows = np.unique(np.r_[0, 1, first - 1, p - start, p - start + 1, T // 3, T - 1].clip(0, T - 1))
+    group = lambda h: slice(h // 7 * HD, (h // 7 + 1) * HD)
+    with np.errstate(all="ignore"):
+        want = attend64(q[rows], k.astype(np.float64), v.astype(np.float64), row_pos[rows], group)
+    for i, t in enumerate(rows):
+        if first <= t < p - start:
+            continue  # in the position's own block
+        for d in range(QD):
+            g, w = got[t, d], want[i, d]
+            if what == "k_nan" and t >= p - start and d >= QD // 2:
+                assert np.isnan(g)
+            elif not np.isfinite(w):
+                assert g == w, (t, d, g, w)
+            else:
+                # Against the dim's own scale: dims differ by tens of decades here.
+                tiny = what == "v_tiny" and d < QD // 2 and d % HD == 9
+                scale = max(abs(w), 1e-36 if tiny else 1.0)
+                assert abs(g - w) <= 1e-5 * scale, (t, d, g, w)
+
+
 @pytest.mark.parametrize("kv", ["f16", "bf16"])
 def test_config5_mixed_step_into_churned_pool(ie, O, dev, kv, impl):
     """BASELINE config 5, both halves of the step: 48 decode sequences (contexts
