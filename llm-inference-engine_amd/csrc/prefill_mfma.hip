@@ -719,6 +719,52 @@ __device__ __forceinline__ void merge_teams(unsigned char* smem, float* out, con
   }
 }
 
+// A block's 16 rows over all their keys with whole float32 operands, on the f32 matrix
+// instruction: for what a row-block kernel's own operands got wrong, by one wave for its dims
+// 16g + 4 wave + e of row r. qv: row r's query times log2(e)/8, [8 ks + j] dim 32 ks + 8g + j.
+// Keys up to `pos` are row r's, up to `last` the block's (V rows past it are taken as zeros).
+template <typename E, typename Page>
+__device__ __forceinline__ f32x4 rows_in_f32(const float (&qv)[16], const char* k_base,
+                                             const char* v_base, size_t page_bytes,
+                                             unsigned row_bytes, Page page, int pos, int last,
+                                             int lane, int wave) {
+  const int g = lane >> 4, r = lane & 15;
+  float top = -INFINITY, total = 0.0f;  // running max, this lane's part of the sum
+  f32x4 x = {0.f, 0.f, 0.f, 0.f};
+#pragma nounroll
+  for (int u = 0; 16 * u <= last; ++u) {
+    const int id = page(u);
+    if (id < 0) continue;
+    const size_t at = size_t(id) * page_bytes;
+    const E* krow = reinterpret_cast<const E*>(k_base + at + r * row_bytes) + 8 * g;
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 16; ++i)  // step i: dim 32 (i/8) + 8g + i%8 of key r
+      s = __builtin_amdgcn_mfma_f32_16x16x4f32(static_cast<float>(krow[32 * (i >> 3) + (i & 7)]), qv[i],
+                                               s, 0, 0, 0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (16 * u + 4 * g + e > pos) s[e] = -INFINITY;
+    const float was = top;
+    top = fmaxf(top, group_max4(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]))));
+    if (top != -INFINITY) {
+      const float corr = exp2_weight(was - top);
+      total *= corr;
+      x *= corr;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {  // step e: key 4g + e, row r of the tile dim 16 (r/4) + 4 wave + r%4
+      const float w = top == -INFINITY ? 0.0f : exp2_weight(s[e] - top);
+      total += w;
+      const E* vrow = reinterpret_cast<const E*>(v_base + at + (4 * g + e) * row_bytes);
+      const float v = 16 * u + 4 * g + e <= last
+                          ? static_cast<float>(vrow[16 * (r >> 2) + 4 * wave + (r & 3)]) : 0.0f;
+      x = __builtin_amdgcn_mfma_f32_16x16x4f32(v, w, x, 0, 0, 0);
+    }
+  }
+  return x * (1.0f / group_sum4(total));
+}
+
 // ---------------------------------------------------------------------------
 // 16-bit caches again, one workgroup per (NB blocks of 16 rows, query head) instead of per
 // (pair of blocks, KV head): its waves take tiles of 16 KT keys in turn, each with its own K
@@ -807,14 +853,11 @@ prefill_rows_kernel(float* __restrict__ out, const float* __restrict__ q,
   // Row r's query of each block, times log2(e)/8: the B operands of S^T (dims 32 ks + 8g ..
   // +7), rotated here when a RoPE table is given (the arithmetic of ie_hip_rope_and_cache;
   // rows outside the table as they are).
-  op qhi[NB][2], qlo[NB][2];
-#pragma unroll
-  for (int b = 0; b < NB; ++b) {
+  auto query = [&](int b, float (&x)[2][8]) {
     const int t = t0 + 16 * b + r;
     const bool row_ok = t < T;
     const float4* src = reinterpret_cast<const float4*>(
         q + (size_t(row_ok ? t : t0) * n_heads + head) * 64 + 8 * g);
-    float x[2][8];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
       const float4 a = src[8 * ks], c = src[8 * ks + 1];
@@ -838,6 +881,12 @@ prefill_rows_kernel(float* __restrict__ out, const float* __restrict__ q,
         x[1][j] = rot ? r1 : x1;
       }
     }
+  };
+  op qhi[NB][2], qlo[NB][2];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    float x[2][8];
+    query(b, x);
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
@@ -1019,8 +1068,23 @@ prefill_rows_kernel(float* __restrict__ out, const float* __restrict__ q,
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) id[kt] = next[kt];
   }
-  merge_teams<NB, kTeams>(smem, out, o, m, lsum, t0, T, n_heads, head, lane, wave,
-                          [](int, f32x4, f32x4*) {});
+  // Blocks before the last: their products take in V rows of the later blocks' positions, with
+  // weight 0, which passes infinities and NaN on. A wave that has written such an output of a
+  // block takes its rows again without them.
+  auto redo = [&](int b, f32x4 y, f32x4* dst) {
+    if (b == NB - 1) return;
+    const int row = t0 + 16 * b + r;
+    const bool odd = !(fabsf(y[0]) + fabsf(y[1]) + (fabsf(y[2]) + fabsf(y[3])) < INFINITY);
+    if (__builtin_amdgcn_ballot_w64(odd && row < T) == 0) return;
+    float x[2][8], qv[16];
+    query(b, x);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) qv[i] = x[i >> 3][i & 7] * (0.125f * kLog2e);
+    y = rows_in_f32<E>(qv, kbase_g, vbase_g, page_bytes, row_bytes, page, pos0 + row,
+                       min(pos0 + t0 + 16 * b + 15, max_pos), lane, wave);
+    if (odd && row < T) *dst = y;
+  };
+  merge_teams<NB, kTeams>(smem, out, o, m, lsum, t0, T, n_heads, head, lane, wave, redo);
 }
 
 // ---------------------------------------------------------------------------
@@ -1292,43 +1356,13 @@ prefill_mfma_f32_kernel(float* __restrict__ out, const float* __restrict__ q,
     for (int e = 0; e < 4; ++e)
       odd |= !(x[e] == 0.0f || (fabsf(x[e]) >= 0x1p-100f && fabsf(x[e]) < INFINITY));
     if (__builtin_amdgcn_ballot_w64(odd && row < T) == 0) return;
-    const float* src = q + (size_t(row < T ? row : t0) * n_heads + head) * 64 + 16 * g;
+    const float* src = q + (size_t(row < T ? row : t0) * n_heads + head) * 64 + 8 * g;
     float qv[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) qv[i] = row < T ? src[i] * (0.125f * kLog2e) : 0.0f;
-    const int last = min(pos0 + t0 + 16 * b + 15, max_pos);
-    float top = -INFINITY, total = 0.0f;  // running max, this lane's part of the sum
-    x = f32x4{0.f, 0.f, 0.f, 0.f};        // row r, dims 16g + 4 wave + e
-#pragma nounroll
-    for (int u = 0; 16 * u <= last; ++u) {
-      const int id = page(u);
-      if (id < 0) continue;
-      const size_t at = size_t(id) * page_bytes;
-      const float* krow = reinterpret_cast<const float*>(kbase_g + at + r * row_bytes) + 16 * g;
-      f32x4 sc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int i = 0; i < 16; ++i)  // step i: dim 16g + i of key r
-        sc = __builtin_amdgcn_mfma_f32_16x16x4f32(krow[i], qv[i], sc, 0, 0, 0);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (16 * u + 4 * g + e > pos0 + row) sc[e] = -INFINITY;
-      const float was = top;
-      top = fmaxf(top, group_max4(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]))));
-      if (top != -INFINITY) {
-        const float corr = exp2_weight(was - top);
-        total *= corr;
-        x *= corr;
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {  // step e: key 4g + e, row r of the tile dim 16 (r/4) + r%4
-        const float w = top == -INFINITY ? 0.0f : exp2_weight(sc[e] - top);
-        total += w;
-        const float* vrow = reinterpret_cast<const float*>(vbase_g + at + (4 * g + e) * row_bytes);
-        const float v = 16 * u + 4 * g + e <= last ? vrow[16 * (r >> 2) + 4 * wave + (r & 3)] : 0.0f;
-        x = __builtin_amdgcn_mfma_f32_16x16x4f32(v, w, x, 0, 0, 0);
-      }
-    }
-    x *= 1.0f / group_sum4(total);
+    for (int i = 0; i < 16; ++i)
+      qv[i] = row < T ? src[32 * (i >> 3) + (i & 7)] * (0.125f * kLog2e) : 0.0f;
+    x = rows_in_f32<float>(qv, kbase_g, vbase_g, page_bytes, row_bytes, page, pos0 + row,
+                           min(pos0 + t0 + 16 * b + 15, max_pos), lane, wave);
     if (row < T) *dst = x;
   };
   merge_teams<NB, kTeams>(smem, out, o, m, l, t0, T, n_heads, head, lane, wave, redo);

@@ -186,6 +186,34 @@ def test_f32_extreme_values(ie, O, dev, what, start, T):
                 assert abs(g - w) <= 1e-5 * scale, (t, d, g, w)
 
 
+@pytest.mark.parametrize("start,T", [(40, 90), (77, 335), (0, 500), (3, 1100), (0, 2800)])
+@pytest.mark.parametrize("kv", ["f16", "bf16"])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_non_finite_value_stays_in_its_rows(ie, O, dev, kv, start, T, bad):
+    """16-bit caches: an infinite or NaN value (an f16 overflow, say) at one of the prompt's own
+    positions does not reach the rows before its block of 16, whatever the work's split, nor
+    the other dims of any row."""
+    kvt = KVS[kv]
+    rng = np.random.default_rng(start + T)
+    n = start + T
+    tables, max_pages, num_pages = make_tables([n], rng)
+    kp, vp = kv_pool(rng, num_pages, kvt, O), kv_pool(rng, num_pages, kvt, O)
+    q, row_pos, row_seq = normal(rng, (T, QD)), np.arange(start, n, dtype=np.int32), np.zeros(T, np.int32)
+    row = T // 64 * 32 + 21
+    rows = np.unique(np.r_[0, row // 16 * 16 - 17, row // 16 * 16 - 16:row // 16 * 16, row, T - 1])
+    want = O.paged_attention(q[rows], kp, vp, kvt, row_pos[rows], row_seq[rows], tables, max_pages,
+                             NH, NKV, HD, threads=8)
+    p = start + row
+    vp[tables[0, p // 16] * 16 + p % 16, 3] = O.round_to_kv(np.array([bad], np.float32), kvt)[0]
+    got = gpu_prefill(ie, dev, q, kp, vp, kvt, row_pos, row_seq, tables, max_pages)[rows]
+    before = rows < row // 16 * 16
+    check(O, got[before], want[before], kvt, "rows before")
+    others = np.ones(QD, bool)
+    others[3:QD // 2:HD] = False  # dim 3 of the query heads on KV head 0
+    check(O, got[:, others], want[:, others], kvt, "other dims")
+    assert not np.isfinite(got[rows >= row][:, ~others]).any()
+
+
 @pytest.mark.parametrize("kv", ["f16", "bf16"])
 def test_config5_mixed_step_into_churned_pool(ie, O, dev, kv, impl):
     """BASELINE config 5, both halves of the step: 48 decode sequences (contexts
