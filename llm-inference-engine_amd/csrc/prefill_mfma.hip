@@ -54,6 +54,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "launch_rules.hpp"
 #include "matmul_tiled.hpp"
 #include "mfma.hpp"
 #include "prefill.hpp"
@@ -773,7 +774,7 @@ __device__ __forceinline__ f32x4 rows_in_f32(const float (&qv)[16], const char* 
 // chip where pairs of blocks x KV heads leave most of it idle. Every wave brings its own K and
 // V (prefill_mfma_kernel's 7 waves share theirs), so long prompts are bound by what a
 // compute unit can take in (4,000 rows: 68 us here, 54 there) and stay there; see
-// launch_prefill_mfma for the line.
+// choose_prefill for the line.
 //   S^T and the softmax as in prefill_mfma_kernel (same operands, rounding and row sums).
 //   O^T[64 dims x 16 rows] += V^T . P^T: row i of tile mt is dim 4i + mt, so lane (g, r)'s
 //     A operand is dim 4r + mt of keys 4g + e of a page pair, and its 8-byte loads of V
@@ -1408,33 +1409,18 @@ int launch_prefill_mfma(float* out, const float* q, const uint16_t* kp, const ui
   const int waves = (group + kHeadsPerWave - 1) / kHeadsPerWave;
   const int n_blocks = (T + kRows - 1) / kRows;
   const dim3 grid((n_blocks + 1) / 2, n_kv_heads);
-  // Which kernel, from the workgroups each would have. A workgroup per (pair of blocks, KV
-  // head) shares every K/V tile among the group's heads, which pays where those workgroups
-  // fill two thirds of the compute units; below, workgroups per (row block, query head).
-  // Measured (us, f16 / bf16; rows on cached positions), pairs of blocks against row blocks:
-  // 4,000 on 0: 54 / 82 against 68 / 95; 2,000 on 0: 31 / 46 against 28 / 34; 2,000 on 2,000:
-  // 67 / 107 against 54 / 73; 600 on 0: 18 / 23 against 11 / 12; 130 on 4,000: 81 / 135 against
-  // 17 / 19. Of the row-block shapes: one block and 8 waves while that gives at most a
-  // workgroup per unit (64 on 2,000, f16: 11.1, two blocks 13); two blocks, 32-key tiles and 8
-  // waves up to 2.5 (512 on 8,000, f16: 37, 4 waves 53); 64-key tiles and 4 waves above
-  // (2,000 on 2,000, bf16: 73, 8 waves 77).
-  const int64_t cus = device_compute_units();
-  if (3 * int64_t(grid.x) * grid.y < 2 * cus) {
-    const int64_t singles = int64_t(n_blocks) * n_heads;
-    const int64_t pairs = (int64_t(T) + 31) / 32 * n_heads;
-    if (singles <= cus)
-      return launch_prefill_rows<KV, 1, 4, 8>(out, q, kp, vp, T, row_pos, row_seq, kv, n_heads,
-                                              n_kv_heads, rope, stream);
-    if (2 * pairs <= 5 * cus)
-      return launch_prefill_rows<KV, 2, 2, 8>(out, q, kp, vp, T, row_pos, row_seq, kv, n_heads,
-                                              n_kv_heads, rope, stream);
+  const bool split = KV == IE_KV_BF16 || prefill_rounding() == IE_HIP_PREFILL_SPLIT;
+  const PrefillKernel kernel = choose_prefill(T, n_heads, n_kv_heads, split, device_compute_units());
+  if (kernel == PrefillKernel::kRows1x8)
+    return launch_prefill_rows<KV, 1, 4, 8>(out, q, kp, vp, T, row_pos, row_seq, kv, n_heads,
+                                            n_kv_heads, rope, stream);
+  if (kernel == PrefillKernel::kRows2x8)
+    return launch_prefill_rows<KV, 2, 2, 8>(out, q, kp, vp, T, row_pos, row_seq, kv, n_heads,
+                                            n_kv_heads, rope, stream);
+  if (kernel == PrefillKernel::kRows2x4)
     return launch_prefill_rows<KV, 2, 4, 4>(out, q, kp, vp, T, row_pos, row_seq, kv, n_heads,
                                             n_kv_heads, rope, stream);
-  }
-  // Two teams splitting the key tiles when the grid alone leaves compute units
-  // without a workgroup or with one: twice the waves per CU, half the serial
-  // tile chain per wave. Larger grids already hold two workgroups per CU.
-  const bool teams2 = int64_t(grid.x) * grid.y <= cus;
+  const bool teams2 = kernel == PrefillKernel::kPairsTwoTeams;
 #define IE_PF_CASE(W)                                                                             \
   case W:                                                                                         \
     return teams2 ? launch_prefill_variant<KV, W, 2>(grid, out, q, kp, vp, T, row_pos, row_seq,   \
@@ -1483,21 +1469,17 @@ int prefill_mfma_launch(float* out, const float* q, const void* k_pool, const vo
       return fail(IE_HIP_EINVAL, "attention_prefill: f32 caches take q rotated by rope_and_cache");
     const float* kf = static_cast<const float*>(k_pool);
     const float* vf = static_cast<const float*>(v_pool);
-    // Two blocks of 16 rows per workgroup halve the splitting of K and V; 8 waves halve a
-    // workgroup's chain of key tiles, 4 leave more of them resident. Measured (us; rows on
-    // cached positions): 2 blocks x 4 waves from 1.75 workgroups per compute unit on (1,333
-    // on 1,000: 73, with 8 waves 82, one block 82); 8 waves below (512 on 8,000: 113, with 4
-    // 142); one block where two leave half the units idle (130 on 4,000: 44, two 57).
-    const int64_t cus = device_compute_units();
-    const int64_t pairs = (int64_t(T) + 31) / 32 * n_heads;
-    if (4 * pairs >= 7 * cus)
-      return launch_prefill_f32<2, 4>(out, q, kf, vf, T, row_pos, row_seq, kv, n_heads, n_kv_heads,
-                                      stream);
-    if (2 * pairs > cus)
-      return launch_prefill_f32<2, 8>(out, q, kf, vf, T, row_pos, row_seq, kv, n_heads, n_kv_heads,
-                                      stream);
-    return launch_prefill_f32<1, 8>(out, q, kf, vf, T, row_pos, row_seq, kv, n_heads, n_kv_heads,
-                                    stream);
+    switch (choose_prefill_f32(T, n_heads, device_compute_units())) {
+      case PrefillKernel::kRows2x4:
+        return launch_prefill_f32<2, 4>(out, q, kf, vf, T, row_pos, row_seq, kv, n_heads, n_kv_heads,
+                                        stream);
+      case PrefillKernel::kRows2x8:
+        return launch_prefill_f32<2, 8>(out, q, kf, vf, T, row_pos, row_seq, kv, n_heads, n_kv_heads,
+                                        stream);
+      default:
+        return launch_prefill_f32<1, 8>(out, q, kf, vf, T, row_pos, row_seq, kv, n_heads, n_kv_heads,
+                                        stream);
+    }
   }
   const uint16_t* kp = static_cast<const uint16_t*>(k_pool);
   const uint16_t* vp = static_cast<const uint16_t*>(v_pool);

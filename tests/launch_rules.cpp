@@ -1,0 +1,11 @@
+// The launch rules (csrc/launch_rules.hpp) behind a C interface, for the CPU tests.
+#include "launch_rules.hpp"
+
+using namespace iehip;
+
+extern "C" int prefill_kernel(int T, int n_heads, int n_kv_heads, int split, int cus) {
+  return int(choose_prefill(T, n_heads, n_kv_heads, split != 0, cus));
+}
+extern "C" int prefill_f32_kernel(int T, int n_heads, int cus) {
+  return int(choose_prefill_f32(T, n_heads, cus));
+}
