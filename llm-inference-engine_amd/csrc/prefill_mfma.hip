@@ -318,11 +318,13 @@ prefill_mfma_kernel(float* __restrict__ out, const float* __restrict__ q,
       }
       // The block's RoPE rows (first segment only; rows outside the table or past
       // the block's rows are not used and stay as they are).
-      if (rope && seg0 == 0 && tid < kRows * 16) {
-        const int ri = tid >> 4, p = pos0 + t0 + ri;
-        if (t0 + ri < T && p >= 0 && p < rope_positions)
-          reinterpret_cast<float4*>(rope_rows + ri * kRopeStride)[tid & 15] =
-              reinterpret_cast<const float4*>(rope + size_t(p) * 64)[tid & 15];
+      if (rope && seg0 == 0) {
+        for (int i = tid; i < kRows * 16; i += 64 * kWaves * kTeams) {
+          const int ri = i >> 4, p = pos0 + t0 + ri;
+          if (t0 + ri < T && p >= 0 && p < rope_positions)
+            reinterpret_cast<float4*>(rope_rows + ri * kRopeStride)[i & 15] =
+                reinterpret_cast<const float4*>(rope + size_t(p) * 64)[i & 15];
+        }
       }
       __syncthreads();
       for (int i = tid; i < n_steps; i += 64 * kWaves * kTeams) {

@@ -8,6 +8,8 @@ import subprocess
 
 import pytest
 
+import test_gpu_prefill_forms as forms
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 CUS = 256
 PAIRS2, PAIRS1, ROWS1X8, ROWS2X8, ROWS2X4 = range(5)
@@ -49,3 +51,13 @@ def test_prefill(rules, T, nh, nkv, single, split):
                                        (2147483647, 14, ROWS2X4)])
 def test_prefill_f32(rules, T, nh, want):
     assert rules.prefill_f32_kernel(T, nh, CUS) == want
+
+
+def test_prefill_forms_are_reached(rules):
+    """The shapes of test_gpu_prefill_forms.py take the forms that they are named after."""
+    got = lambda T, nh, nkv: {rules.prefill_kernel(T, nh, nkv, split, CUS) for split in (0, 1)}
+    assert all(got(*s) == {PAIRS2} for s in forms.PAIRS_TWO_TEAMS + [forms.SEGMENTS_TWO_TEAMS[1:]])
+    assert all(got(*s) == {PAIRS1} for s in forms.PAIRS_ONE_TEAM + [forms.SEGMENTS_ONE_TEAM[1:]])
+    assert got(*forms.ONE_TILE_OF_TWO_BLOCKS) == {ROWS2X8}
+    for shapes in (forms.PAIRS_TWO_TEAMS, forms.PAIRS_ONE_TEAM):
+        assert {nh // nkv for _, nh, nkv in shapes} == set(range(1, 9))
