@@ -677,13 +677,32 @@ inline int64_t unit_grid(int64_t n_units, int n_heads, int n_kv_heads, int threa
 
 // The waves' (o, m, l) through LDS (their stages are idle: no DMA is left in flight) and the
 // output: wave w < 4 finishes row r's dims 16g + 4w .. +3. l is the row's whole sum, in every
-// lane; o[b][mt][t] is dim 16g + 4t + mt. after(b, x, dst) follows block b's result x into `out`.
+// lane; o[b][mt][t] is dim 16g + 4t + mt. after(b, w, x, dst) follows dims
+// 16g + 4w .. of block b's result x into `out`.
+// n_tiles == 1: only wave 0 took keys, and writes its own result (32/8 heads, 2 rows: 5.7 us
+// through the merge, 4.7, by pairs 5.3). The f32 kernel, which has no registers to spare for that, gives kTeams.
 template <int NB, int kTeams, typename After>
 __device__ __forceinline__ void merge_teams(unsigned char* smem, float* out, const f32x4 (&o)[NB][4],
                                             const float (&m)[NB], const float (&l)[NB], int t0,
                                             int T, int n_heads, int head, int lane, int wave,
-                                            After after) {
+                                            int n_tiles, After after) {
   const int g = lane >> 4, r = lane & 15;
+  if (n_tiles == 1) {  // wave 0 has it all
+    if (wave > 0) return;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int t = t0 + 16 * b + r;
+      f32x4* const dst = reinterpret_cast<f32x4*>(out + (size_t(t) * n_heads + head) * 64 + 16 * g);
+      const float il = 1.0f / l[b];
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const f32x4 x = f32x4{o[b][0][w], o[b][1][w], o[b][2][w], o[b][3][w]} * il;
+        if (t < T) dst[w] = x;
+        after(b, w, x, dst + w);
+      }
+    }
+    return;
+  }
   __syncthreads();
   f32x4* const xo = reinterpret_cast<f32x4*>(smem);                          // [wave][b][t][lane]
   float2* const xml = reinterpret_cast<float2*>(smem + kTeams * NB * 4096);  // [wave][b][lane]
@@ -718,19 +737,19 @@ __device__ __forceinline__ void merge_teams(unsigned char* smem, float* out, con
         reinterpret_cast<f32x4*>(out + (size_t(t) * n_heads + head) * 64 + 16 * g + 4 * wave);
     const f32x4 x = sum * (1.0f / total);
     if (t < T) *dst = x;
-    after(b, x, dst);
+    after(b, wave, x, dst);
   }
 }
 
 // A block's 16 rows over all their keys with whole float32 operands, on the f32 matrix
-// instruction: for what a row-block kernel's own operands got wrong, by one wave for its dims
-// 16g + 4 wave + e of row r. qv: row r's query times log2(e)/8, [8 ks + j] dim 32 ks + 8g + j.
+// instruction: for what a row-block kernel's own operands got wrong, by one wave for dims
+// 16g + 4 part + e of row r. qv: row r's query times log2(e)/8, [8 ks + j] dim 32 ks + 8g + j.
 // Keys up to `pos` are row r's, up to `last` the block's (V rows past it are taken as zeros).
 template <typename E, typename Page>
 __device__ __forceinline__ f32x4 rows_in_f32(const float (&qv)[16], const char* k_base,
                                              const char* v_base, size_t page_bytes,
                                              unsigned row_bytes, Page page, int pos, int last,
-                                             int lane, int wave) {
+                                             int lane, int part) {
   const int g = lane >> 4, r = lane & 15;
   float top = -INFINITY, total = 0.0f;  // running max, this lane's part of the sum
   f32x4 x = {0.f, 0.f, 0.f, 0.f};
@@ -756,12 +775,12 @@ __device__ __forceinline__ f32x4 rows_in_f32(const float (&qv)[16], const char* 
       x *= corr;
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {  // step e: key 4g + e, row r of the tile dim 16 (r/4) + 4 wave + r%4
+    for (int e = 0; e < 4; ++e) {  // step e: key 4g + e, row r of the tile dim 16 (r/4) + 4 part + r%4
       const float w = top == -INFINITY ? 0.0f : exp2_weight(s[e] - top);
       total += w;
       const E* vrow = reinterpret_cast<const E*>(v_base + at + (4 * g + e) * row_bytes);
       const float v = 16 * u + 4 * g + e <= last
-                          ? static_cast<float>(vrow[16 * (r >> 2) + 4 * wave + (r & 3)]) : 0.0f;
+                          ? static_cast<float>(vrow[16 * (r >> 2) + 4 * part + (r & 3)]) : 0.0f;
       x = __builtin_amdgcn_mfma_f32_16x16x4f32(v, w, x, 0, 0, 0);
     }
   }
@@ -1074,7 +1093,7 @@ prefill_rows_kernel(float* __restrict__ out, const float* __restrict__ q,
   // Blocks before the last: their products take in V rows of the later blocks' positions, with
   // weight 0, which passes infinities and NaN on. A wave that has written such an output of a
   // block takes its rows again without them.
-  auto redo = [&](int b, f32x4 y, f32x4* dst) {
+  auto redo = [&](int b, int part, f32x4 y, f32x4* dst) {
     if (b == NB - 1) return;
     const int row = t0 + 16 * b + r;
     const bool odd = !(fabsf(y[0]) + fabsf(y[1]) + (fabsf(y[2]) + fabsf(y[3])) < INFINITY);
@@ -1084,10 +1103,10 @@ prefill_rows_kernel(float* __restrict__ out, const float* __restrict__ q,
 #pragma unroll
     for (int i = 0; i < 16; ++i) qv[i] = x[i >> 3][i & 7] * (0.125f * kLog2e);
     y = rows_in_f32<E>(qv, kbase_g, vbase_g, page_bytes, row_bytes, page, pos0 + row,
-                       min(pos0 + t0 + 16 * b + 15, max_pos), lane, wave);
+                       min(pos0 + t0 + 16 * b + 15, max_pos), lane, part);
     if (odd && row < T) *dst = y;
   };
-  merge_teams<NB, kTeams>(smem, out, o, m, lsum, t0, T, n_heads, head, lane, wave, redo);
+  merge_teams<NB, kTeams>(smem, out, o, m, lsum, t0, T, n_heads, head, lane, wave, n_tiles, redo);
 }
 
 // ---------------------------------------------------------------------------
@@ -1352,7 +1371,7 @@ prefill_mfma_f32_kernel(float* __restrict__ out, const float* __restrict__ q,
   // keys again with the whole float32 values, on the f32 instruction, for its own 16 dims.
   // (Looked for after the write: no size is slower by more than 2%; every wave looking at its
   // own sums before the merge took 1.4 us more a launch.)
-  auto redo = [&](int b, f32x4 x, f32x4* dst) {
+  auto redo = [&](int b, int part, f32x4 x, f32x4* dst) {
     const int row = t0 + 16 * b + r;
     bool odd = false;
 #pragma unroll
@@ -1365,10 +1384,10 @@ prefill_mfma_f32_kernel(float* __restrict__ out, const float* __restrict__ q,
     for (int i = 0; i < 16; ++i)
       qv[i] = row < T ? src[32 * (i >> 3) + (i & 7)] * (0.125f * kLog2e) : 0.0f;
     x = rows_in_f32<float>(qv, kbase_g, vbase_g, page_bytes, row_bytes, page, pos0 + row,
-                           min(pos0 + t0 + 16 * b + 15, max_pos), lane, wave);
+                           min(pos0 + t0 + 16 * b + 15, max_pos), lane, part);
     if (row < T) *dst = x;
   };
-  merge_teams<NB, kTeams>(smem, out, o, m, l, t0, T, n_heads, head, lane, wave, redo);
+  merge_teams<NB, kTeams>(smem, out, o, m, l, t0, T, n_heads, head, lane, wave, kTeams, redo);
 }
 
 template <int NB, int kTeams>
