@@ -464,6 +464,10 @@ decode_partial_mfma(float* __restrict__ out, float* __restrict__ part_o,
     // result by fold_pair. Each pair's partial depends on the pair alone, so a
     // chunk's result is the same whether one wave folds its pairs as they come
     // or several waves take one pair each and one of them folds the others'.
+    f32x4 sc[2] = {sa, sb};
+    settle(sc);
+    sa = sc[0];
+    sb = sc[1];
     float mx = max_nn(max3_nn(sa[0], sa[1], sa[2]),
                       max3_nn(max3_nn(sa[3], sb[0], sb[1]), sb[2], sb[3]));
     mx = group_max4(mx);

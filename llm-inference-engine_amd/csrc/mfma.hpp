@@ -129,17 +129,18 @@ __device__ __forceinline__ float max3_nn(float a, float b, float c) {
   asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
   return r;
 }
-// The wait states (at most 11 for the instructions used here) between a matrix instruction
-// and inline assembly that reads its result, or that is given a register of a result
-// nothing reads: a VALU instruction inside assembly would read the registers as they were
-// before, or have what it wrote replaced by the result that arrives after it.
+// The wait states (8 after a 16x16x32 product, as the compiler itself places) between a matrix
+// instruction and inline assembly that reads its result, or that is given a register of a
+// result nothing reads: a VALU instruction inside assembly would read the registers as they
+// were before, or have what it wrote replaced by the result that arrives after it. Tests look
+// through the built library's instructions for any such pair.
 template <int N>
 __device__ __forceinline__ void settle(f32x4 (&x)[N]) {
   static_assert(N >= 1 && N <= 4, "accumulators of one wave tile");
-  if constexpr (N == 1) asm volatile("s_nop 11" : "+v"(x[0]));
-  if constexpr (N == 2) asm volatile("s_nop 11" : "+v"(x[0]), "+v"(x[1]));
-  if constexpr (N == 3) asm volatile("s_nop 11" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]));
-  if constexpr (N == 4) asm volatile("s_nop 11" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]));
+  if constexpr (N == 1) asm volatile("s_nop 7" : "+v"(x[0]));
+  if constexpr (N == 2) asm volatile("s_nop 7" : "+v"(x[0]), "+v"(x[1]));
+  if constexpr (N == 3) asm volatile("s_nop 7" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]));
+  if constexpr (N == 4) asm volatile("s_nop 7" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]));
 }
 
 __device__ __forceinline__ float group_max4(float x) {

@@ -440,6 +440,7 @@ prefill_mfma_kernel(float* __restrict__ out, const float* __restrict__ q,
 #pragma unroll
           for (int hh = 0; hh < kHeadsPerWave; ++hh) {
             auto raise = [&]() {
+              settle(s[hh]);
               const f32x4(&sh)[4] = s[hh];
               float mx = max_nn(max3_nn(max3_nn(sh[0][0], sh[0][1], sh[0][2]),
                                         max3_nn(sh[0][3], sh[1][0], sh[1][1]),
