@@ -23,9 +23,9 @@
 // Lane (g, r) of a tile: A = W[row r][k + 8g .. +8], B = x[token r][k + 8g ..
 // +8]; the result lane holds rows 4g .. 4g+3 of token r.
 #include <algorithm>
-#include <iterator>
 
 #include "common.hpp"
+#include "launch_rules.hpp"
 #include "matmul_tiled.hpp"
 #include "mfma.hpp"
 
@@ -263,23 +263,6 @@ int check_matrix(const ie_matrix& m, const char* who) {
   return IE_HIP_OK;
 }
 
-// The LDS-tiled kernel's launch. A tile shape is chosen by the time its launch should take:
-// rounds over the compute units times a workgroup's time, which is a fixed part plus a part
-// per K block of a slot. The parts (ns) were fitted on an MI355X to o_proj (896 x 896) and
-// down (896 x 4,864) with at most one workgroup per compute unit, launch overhead taken
-// off; the choice was then within 8% of the fastest shape for q/k/v, o_proj, gate/up and
-// down at 21 batch sizes from 1 to 4,000 tokens. What the shapes gain over one 16- or
-// 32-row tile per workgroup at every size (us, bf16): gate/up 16.3 -> 12.1 at 64 tokens,
-// 104 -> 44 at 600, 630 -> 252 at 4,000; down 11.1 -> 8.7, 47 -> 27, 246 -> 123.
-struct Tile {
-  int nr, ct, w;           // row tiles (of all weight matrices) and token tiles, waves
-  int fixed_ns, block_ns;  // a workgroup's time: fixed + block * (K blocks of a slot)
-};
-constexpr Tile kPlainTiles[] = {{1, 1, 8, 600, 280},  {2, 1, 8, 750, 390},  {2, 2, 8, 700, 620},
-                                {3, 2, 4, 1300, 900}, {4, 2, 4, 1600, 940}, {6, 2, 4, 2000, 1210},
-                                {8, 2, 4, 2500, 1470}};
-constexpr Tile kGateTiles[] = {{2, 1, 8, 750, 390}, {4, 1, 8, 700, 680}, {4, 2, 8, 1000, 850},
-                               {6, 2, 4, 2000, 1210}, {8, 2, 4, 2500, 1470}};
 constexpr int kTiledMaxLds = 160 * 1024;  // a gfx950 compute unit's LDS
 
 // One launch of a tile shape; false (nothing launched) where its LDS or its grid does not fit.
@@ -368,43 +351,18 @@ struct TiledLaunch {
     *rc = IE_HIP_OK;
     return true;
   }
-  // Wide matrices (4 slots, one wave each). Up to 64 tokens with K up to 1,024 (8 blocks a
-  // slot, held in registers) the weights are streamed past the tokens, except for 17 to 32
-  // tokens, where 128 x 32 tiles take as long and spill nothing. The 151,936-row LM head, us,
-  // direct loads before / tiles / streamed: bf16, 1 token 59 / 52 / 49, 16 tokens 74 / 64 /
-  // 57, 32 tokens 90 / 65 / 63, 64 tokens 138 / 92 / 76; INT8, 1 token 58 / 36 / 34, 16 tokens
-  // 65 / 43 / 39, 64 tokens 177 / 73 / 64. (HBM's share, at the 5.1 TB/s of a large copy:
-  // bf16 53 to 61, INT8 27 to 34.)
+  // Wide matrices (4 slots, one wave each).
   bool run_wide(bool gate, int* rc) const {
-    if (gate) return with_types<true, 8, 2, 4, 4, 1>(rc);
-    if (w->cols <= 32 * 4 * 8) {
-      if (T <= 16)
+    switch (choose_wide(gate, w->cols, T)) {
+      case WideKernel::kGateTiles: return with_types<true, 8, 2, 4, 4, 1>(rc);
+      case WideKernel::kTiles16: return with_types<false, 4, 1, 4, 4, 2>(rc);
+      case WideKernel::kTiles32: return with_types<false, 8, 2, 4, 4, 1>(rc);
+      case WideKernel::kStream16:
         return w->int8 ? stream_go<4, 1, 1, true>(2, rc) : stream_go<2, 1, 1, false>(1, rc);
-      if (T > 32 && T <= 64)
-        return w->int8 ? stream_go<2, 2, 2, true>(1, rc) : stream_go<2, 2, 2, false>(1, rc);
+      default: return w->int8 ? stream_go<2, 2, 2, true>(1, rc) : stream_go<2, 2, 2, false>(1, rc);
     }
-    return T <= 16 ? with_types<false, 4, 1, 4, 4, 2>(rc) : with_types<false, 8, 2, 4, 4, 1>(rc);
   }
 };
-
-int choose_tile(bool gate, int rows, int cols, int T, int cus) {
-  const Tile* tiles = gate ? kGateTiles : kPlainTiles;
-  const int count = gate ? int(std::size(kGateTiles)) : int(std::size(kPlainTiles));
-  const int64_t blocks = (cols / 32 + 7) / 8;
-  int best = 0;
-  int64_t best_ns = INT64_MAX;
-  for (int i = 0; i < count; ++i) {
-    const Tile& t = tiles[i];
-    const int64_t rt = 16 * (gate ? t.nr / 2 : t.nr), tt = 16 * t.ct;
-    const int64_t groups = ((rows + rt - 1) / rt) * ((T + tt - 1) / tt);
-    const int64_t ns = ((groups + cus - 1) / cus) * (t.fixed_ns + t.block_ns * blocks);
-    if (ns < best_ns) {
-      best_ns = ns;
-      best = i;
-    }
-  }
-  return best;
-}
 
 int launch_matmul(bool gate, float* y, const float* x, const ie_matrix& w, const ie_matrix* w2,
                   const float* bias, int T, int accumulate, hipStream_t stream, const char* who,

@@ -3,6 +3,7 @@
 #pragma once
 
 #include <cstdint>
+#include <iterator>
 
 namespace iehip {
 
@@ -52,6 +53,60 @@ inline PrefillKernel choose_prefill_f32(int T, int n_heads, int64_t cus) {
   const int64_t pairs = (int64_t(T) + 31) / 32 * n_heads;
   if (4 * pairs >= 7 * cus) return PrefillKernel::kRows2x4;
   return 2 * pairs > cus ? PrefillKernel::kRows2x8 : PrefillKernel::kRows1x8;
+}
+
+// The projections' LDS tiles (matmul_tiled_kernel). A shape is chosen by the time its launch should take:
+// rounds over the compute units times a workgroup's time, which is a fixed part plus a part
+// per K block of a slot. The parts (ns) were fitted on an MI355X to o_proj (896 x 896) and
+// down (896 x 4,864) with at most one workgroup per compute unit, launch overhead taken
+// off; the choice was then within 8% of the fastest shape for q/k/v, o_proj, gate/up and
+// down at 21 batch sizes from 1 to 4,000 tokens. What the shapes gain over one 16- or
+// 32-row tile per workgroup at every size (us, bf16): gate/up 16.3 -> 12.1 at 64 tokens,
+// 104 -> 44 at 600, 630 -> 252 at 4,000; down 11.1 -> 8.7, 47 -> 27, 246 -> 123.
+struct Tile {
+  int nr, ct, w;           // row tiles (of all weight matrices) and token tiles, waves
+  int fixed_ns, block_ns;  // a workgroup's time: fixed + block * (K blocks of a slot)
+};
+constexpr Tile kPlainTiles[] = {{1, 1, 8, 600, 280},  {2, 1, 8, 750, 390},  {2, 2, 8, 700, 620},
+                                {3, 2, 4, 1300, 900}, {4, 2, 4, 1600, 940}, {6, 2, 4, 2000, 1210},
+                                {8, 2, 4, 2500, 1470}};
+constexpr Tile kGateTiles[] = {{2, 1, 8, 750, 390}, {4, 1, 8, 700, 680}, {4, 2, 8, 1000, 850},
+                               {6, 2, 4, 2000, 1210}, {8, 2, 4, 2500, 1470}};
+inline int choose_tile(bool gate, int rows, int cols, int T, int cus) {
+  const Tile* tiles = gate ? kGateTiles : kPlainTiles;
+  const int count = gate ? int(std::size(kGateTiles)) : int(std::size(kPlainTiles));
+  const int64_t blocks = (cols / 32 + 7) / 8;
+  int best = 0;
+  int64_t best_ns = INT64_MAX;
+  for (int i = 0; i < count; ++i) {
+    const Tile& t = tiles[i];
+    const int64_t rt = 16 * (gate ? t.nr / 2 : t.nr), tt = 16 * t.ct;
+    const int64_t groups = ((rows + rt - 1) / rt) * ((T + tt - 1) / tt);
+    const int64_t ns = ((groups + cus - 1) / cus) * (t.fixed_ns + t.block_ns * blocks);
+    if (ns < best_ns) {
+      best_ns = ns;
+      best = i;
+    }
+  }
+  return best;
+}
+
+// Wide matrices (16 row tiles per compute unit: LM heads): tiles of 64 rows x 16 tokens or
+// 128 x 32, or their weights streamed past up to 16 or 64 tokens whose split activations stay
+// in registers (K up to 1,024). The stream counts 8 K blocks per slot whatever there are, so it
+// pays where K comes near that: from 768 columns at 33 to 64 tokens, 896 at up to 16; at 17 to
+// 32, 128 x 32 tiles take as long and spill nothing. The 151,936-row LM head with 896 columns,
+// us, direct loads before / tiles / streamed: bf16, 1 token 59 / 52 / 49, 16 tokens 74 / 64 / 57,
+// 32 tokens 90 / 65 / 63, 64 tokens 138 / 92 / 76; INT8, 1 token 58 / 36 / 34, 16 tokens 65 /
+// 43 / 39, 64 tokens 177 / 73 / 64. (HBM's share, at the 5.1 TB/s of a large copy: bf16 53 to 61,
+// INT8 27 to 34.) With 512 columns, tiles / streamed: bf16, 16 tokens 26.5 / 31.9, 64 tokens
+// 45.6 / 53.2; with 128: 12.5 / 26.8 and 24.9 / 47.8 (direct loads 15.8 and 42.6).
+enum class WideKernel { kGateTiles, kTiles16, kTiles32, kStream16, kStream64 };
+inline WideKernel choose_wide(bool gate, int cols, int T) {
+  if (gate) return WideKernel::kGateTiles;
+  if (T <= 16) return cols >= 896 && cols <= 1024 ? WideKernel::kStream16 : WideKernel::kTiles16;
+  return T > 32 && T <= 64 && cols >= 768 && cols <= 1024 ? WideKernel::kStream64
+                                                          : WideKernel::kTiles32;
 }
 
 }  // namespace iehip

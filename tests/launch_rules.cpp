@@ -9,3 +9,7 @@ extern "C" int prefill_kernel(int T, int n_heads, int n_kv_heads, int split, int
 extern "C" int prefill_f32_kernel(int T, int n_heads, int cus) {
   return int(choose_prefill_f32(T, n_heads, cus));
 }
+extern "C" int tile(int gate, int rows, int cols, int T, int cus) {
+  return choose_tile(gate != 0, rows, cols, T, cus);
+}
+extern "C" int wide_kernel(int gate, int cols, int T) { return int(choose_wide(gate != 0, cols, T)); }

@@ -289,12 +289,14 @@ def test_dense_argument_errors(ie, dev):
 
 
 # T, rows, cols: every LDS tile shape with ragged edges (rows % 16, rows % 4, T % 16 and the K
-# blocks' share per slot all uneven), the smallest K that takes LDS tiles and the one below it,
-# and wide matrices streamed past 16 and 64 tokens, up to the K and tokens where that ends.
+# blocks' share per slot all uneven), K below a block per slot, and wide matrices in tiles of 16
+# and 32 tokens and streamed past 16 and 64, up to the K and tokens where that ends
+# (test_launch_rules.py checks that these shapes take every form).
 TILED = [(1, 898, 288), (17, 898, 288), (77, 898, 288), (200, 898, 288), (333, 898, 288),
          (600, 898, 288), (1003, 898, 288), (450, 1152, 896), (50, 900, 256), (50, 900, 224),
          (9, 70001, 128), (21, 70001, 160), (16, 70001, 992), (17, 65537, 1024), (33, 70001, 224),
-         (64, 65540, 1024), (40, 66000, 1056), (65, 66000, 896)]
+         (64, 65540, 1024), (40, 66000, 1056), (65, 66000, 896), (450, 898, 288), (9, 70001, 928),
+         (33, 70001, 800)]
 
 
 @pytest.mark.parametrize("T,rows,cols", TILED)
@@ -321,7 +323,8 @@ def test_tile_shapes(ie, dev, T, rows, cols, int8):
 @pytest.mark.parametrize("T", [1, 20, 40, 90, 300])
 @pytest.mark.parametrize("int8", [False, True])
 def test_gate_tile_shapes(ie, dev, T, int8):
-    """The gate/up form of each shape, with and without the folded rmsnorm, at 4,866 rows."""
+    """The gate/up form at 4,866 rows (32 rows of both matrices x 16 and 32 tokens), with and
+    without the folded rmsnorm."""
     rng = np.random.default_rng(T)
     rows, cols = 4866, 288
     x = rng.standard_normal((T, cols), dtype=np.float32)
@@ -337,3 +340,37 @@ def test_gate_tile_shapes(ie, dev, T, int8):
         torch.cuda.synchronize()
         g, u = (O.matmul(xin, w, fmt, s, None) for _, _, (w, fmt, s) in ws)
         assert rel_err(out.cpu().numpy(), O.silu_mul(g, u)) <= REL
+
+
+# T, rows, cols: every gate/up tile shape with ragged rows (48 rows of two INT8 matrices straddle
+# one 1 KB load), and wide matrices.
+GATE_TILED = [(1, 898, 288), (77, 898, 288), (150, 898, 288), (333, 898, 288), (450, 898, 896),
+              (5, 65530, 160), (37, 65537, 96)]
+
+
+@pytest.mark.parametrize("T,rows,cols", GATE_TILED)
+@pytest.mark.parametrize("int8", [False, True])
+def test_gate_tiles(ie, dev, T, rows, cols, int8):
+    """Against the oracle, and the first and last token bit for bit what they are alone; with the
+    folded rmsnorm too, which wide matrices do not take."""
+    rng = np.random.default_rng(T + rows)
+    x = rng.standard_normal((T, cols), dtype=np.float32)
+    ws = [dev_weights(ie, dev, rng.standard_normal((rows, cols), dtype=np.float32) * np.float32(0.1),
+                      int8) for _ in range(2)]
+    wn = rng.standard_normal(cols, dtype=np.float32)
+    dx, dn = torch.from_numpy(x).to(dev), torch.from_numpy(wn).to(dev)
+    forms = [(x, lambda o, a: ie.gate_up_silu(o, a, ws[0][0], ws[1][0]))]
+    if rows < 65000:
+        forms.append((O.rmsnorm(x, wn, 1e-6),
+                      lambda o, a: ie.rmsnorm_gate_up_silu(o, a, dn, 1e-6, ws[0][0], ws[1][0])))
+    for xin, call in forms:
+        out = torch.full((T, rows), float("nan"), device=dev)
+        one = torch.empty((1, rows), device=dev)
+        call(out, dx)
+        torch.cuda.synchronize()
+        g, u = (O.matmul(xin, w, fmt, s, None) for _, _, (w, fmt, s) in ws)
+        assert rel_err(out.cpu().numpy(), O.silu_mul(g, u)) <= REL
+        for t in (0, T - 1):
+            call(one, dx[t:t + 1].contiguous())
+            torch.cuda.synchronize()
+            assert torch.equal(one[0].view(torch.int32), out[t].view(torch.int32)), t

@@ -8,11 +8,13 @@ import subprocess
 
 import pytest
 
+import test_gpu_dense as dense
 import test_gpu_prefill_forms as forms
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CUS = 256
 PAIRS2, PAIRS1, ROWS1X8, ROWS2X8, ROWS2X4 = range(5)
+GATE_TILES, TILES16, TILES32, STREAM16, STREAM64 = range(5)
 
 
 @pytest.fixture(scope="session")
@@ -61,3 +63,28 @@ def test_prefill_forms_are_reached(rules):
     assert got(*forms.ONE_TILE_OF_TWO_BLOCKS) == {ROWS2X8}
     for shapes in (forms.PAIRS_TWO_TEAMS, forms.PAIRS_ONE_TEAM):
         assert {nh // nkv for _, nh, nkv in shapes} == set(range(1, 9))
+
+
+@pytest.mark.parametrize("cols,T,want", [
+    (896, 1, STREAM16), (896, 16, STREAM16), (1024, 16, STREAM16), (1056, 16, TILES16),
+    (864, 16, TILES16), (128, 1, TILES16), (896, 17, TILES32), (896, 32, TILES32),
+    (896, 33, STREAM64), (768, 64, STREAM64), (1024, 64, STREAM64), (736, 64, TILES32),
+    (128, 64, TILES32), (1056, 64, TILES32), (896, 65, TILES32)])
+def test_wide(rules, cols, T, want):
+    """LM heads: the weights are streamed where K fills the registers that are set aside for it."""
+    assert rules.wide_kernel(0, cols, T) == want
+    assert rules.wide_kernel(1, cols, T) == GATE_TILES
+
+
+def test_dense_shapes_are_reached(rules):
+    """test_gpu_dense.py's shapes take every tile shape and every wide form, with ragged rows."""
+    wide = lambda rows: (rows + 15) // 16 >= 16 * CUS
+    plain = {rules.tile(0, rows, cols, T, CUS) for T, rows, cols in dense.TILED
+             if not wide(rows) and cols >= 256 and rows % 16}
+    assert plain == set(range(7))
+    gate = {rules.tile(1, rows, cols, T, CUS) for T, rows, cols in dense.GATE_TILED
+            if not wide(rows) and cols >= 256 and rows % 16}
+    assert gate == set(range(5))
+    forms = {rules.wide_kernel(0, cols, T) for T, rows, cols in dense.TILED if wide(rows)}
+    assert forms == {TILES16, TILES32, STREAM16, STREAM64}
+    assert any(wide(rows) for _, rows, _ in dense.GATE_TILED)
