@@ -265,7 +265,8 @@ int check_matrix(const ie_matrix& m, const char* who) {
 
 constexpr int kTiledMaxLds = 160 * 1024;  // a gfx950 compute unit's LDS
 
-// One launch of a tile shape; false (nothing launched) where its LDS or its grid does not fit.
+// One launch of a tile shape; false (nothing launched) where its LDS, its grid or its offsets do
+// not fit.
 struct TiledLaunch {
   float* y;
   const float* x;
@@ -285,7 +286,9 @@ struct TiledLaunch {
     const int64_t lds = int64_t(Shape::kLds) + (NORM ? int64_t(w->cols) * 4 : 0);
     const int64_t row_tiles = (int64_t(w->rows) + Shape::kRows - 1) / Shape::kRows;
     const int64_t tok_tiles = (int64_t(T) + Shape::kTokens - 1) / Shape::kTokens;
-    if (lds > kTiledMaxLds || row_tiles * tok_tiles * 64 * W > int64_t(UINT32_MAX)) return false;
+    if (lds > kTiledMaxLds || row_tiles * tok_tiles * 64 * W > int64_t(UINT32_MAX) ||
+        !tile_offsets_fit(Shape::kRows, Shape::kTokens, w->cols, I8 ? 1 : 2))
+      return false;
     const auto kernel = matmul_tiled_kernel<GATE, RT, CT, W, SLOTS, S, I8, NORM>;
     if (lds > 64 * 1024) {  // above the default dynamic-LDS cap
       static const hipError_t attr =

@@ -91,6 +91,13 @@ inline int choose_tile(bool gate, int rows, int cols, int T, int cus) {
   return best;
 }
 
+// Whether a tile's byte offsets from its first row and token fit the 32 bits that its loads
+// take them in (128 bf16 rows: up to 16.7 M columns).
+inline bool tile_offsets_fit(int tile_rows, int tile_tokens, int64_t cols, int weight_bytes) {
+  return tile_rows * cols * weight_bytes <= int64_t(UINT32_MAX) &&
+         tile_tokens * cols * 4 <= int64_t(UINT32_MAX);
+}
+
 // Wide matrices (16 row tiles per compute unit: LM heads): tiles of 64 rows x 16 tokens or
 // 128 x 32, or their weights streamed past up to 16 or 64 tokens whose split activations stay
 // in registers (K up to 1,024). The stream counts 8 K blocks per slot whatever there are, so it

@@ -218,7 +218,7 @@ matmul_tiled_kernel(float* __restrict__ y, const float* __restrict__ x, const vo
   // bf16, load u is row tile u, lane l row l/4, 16-byte piece (l%4) ^ (row/2 % 4); int8,
   // load u is row tiles 2u and 2u + 1, lane l row l/2 of the 32, piece (l%2) ^ (row/4 % 2).
   // Activations: load p is tokens 8p .. 8p+7, lane l token l/8, piece (l%8) ^ (l/8). LDS
-  // slot = lane. (The host keeps a tile's offsets within 32 bits.)
+  // slot = lane. (The host takes this kernel where a tile's offsets fit 32 bits: tile_offsets_fit.)
   constexpr int kWBytes = I8 ? 1 : 2;
   const int wr = I8 ? lane >> 1 : lane >> 2;
   const int wp = I8 ? (lane & 1) ^ ((wr >> 2) & 1) : (lane & 3) ^ ((wr >> 1) & 3);

@@ -374,3 +374,21 @@ def test_gate_tiles(ie, dev, T, rows, cols, int8):
             call(one, dx[t:t + 1].contiguous())
             torch.cuda.synchronize()
             assert torch.equal(one[0].view(torch.int32), out[t].view(torch.int32)), t
+
+
+def test_offsets_past_32_bits(ie, dev):
+    """Rows of 150 M columns: the last of 16 lies more than 4 GB behind the first, so LDS tiles,
+    whose loads take 32-bit offsets, are not chosen. Small whole numbers: every sum is exact."""
+    rows, cols = 16, 150_000_000
+    at = torch.tensor([0, 5, 31, 32, 4_097, 70_000_007, cols - 33, cols - 1])
+    w = torch.zeros((rows, cols), dtype=torch.bfloat16, device=dev)
+    w[:, at.to(dev)] = (torch.arange(rows)[:, None] + torch.arange(len(at))[None, :] + 1).to(dev).bfloat16()
+    x = torch.zeros((1, cols), device=dev)
+    x[0, at.to(dev)] = torch.arange(1.0, len(at) + 1, device=dev)
+    y = torch.empty((1, rows), device=dev)
+    ie.matmul(y, x, ie.matrix(w))
+    torch.cuda.synchronize()
+    want = [sum((r + i + 1) * (i + 1) for i in range(len(at))) for r in range(rows)]
+    assert y[0].tolist() == want
+    del w, x
+    torch.cuda.empty_cache()

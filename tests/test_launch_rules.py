@@ -88,3 +88,14 @@ def test_dense_shapes_are_reached(rules):
     forms = {rules.wide_kernel(0, cols, T) for T, rows, cols in dense.TILED if wide(rows)}
     assert forms == {TILES16, TILES32, STREAM16, STREAM64}
     assert any(wide(rows) for _, rows, _ in dense.GATE_TILED)
+
+
+@pytest.mark.parametrize("rows,tokens,cols,wbytes,fits", [
+    (128, 32, 16_777_184, 2, 1), (128, 32, 16_777_216, 2, 0), (128, 32, 33_554_400, 1, 1),
+    (128, 32, 33_554_432, 1, 0), (16, 16, 67_108_832, 2, 1), (16, 16, 67_108_864, 2, 0),
+    (16, 16, 150_000_000, 2, 0), (16, 16, 2_147_483_616, 2, 0)])
+def test_tile_offsets(rules, rows, tokens, cols, wbytes, fits):
+    """The last byte of a tile's last row and token is within 32 bits of its first, or the
+    launch goes to the kernel with 64-bit addresses."""
+    assert rules.offsets_fit(rows, tokens, ctypes.c_int64(cols), wbytes) == fits
+    assert fits == (rows * cols * wbytes < 2**32 and tokens * cols * 4 < 2**32)
