@@ -279,7 +279,7 @@ struct TiledLaunch {
   int vec;
   hipStream_t stream;
 
-  template <bool GATE, int NR, int CT, int W, int SLOTS, int S, bool I8, bool NORM>
+  template <bool GATE, int NR, int CT, int W, int SLOTS, int S, bool I8, bool NORM, bool SHORT>
   bool go(int* rc) const {
     constexpr int RT = NR / (GATE ? 2 : 1);
     using Shape = TiledShape<GATE, RT, CT, W, S, I8>;
@@ -289,7 +289,7 @@ struct TiledLaunch {
     if (lds > kTiledMaxLds || row_tiles * tok_tiles * 64 * W > int64_t(UINT32_MAX) ||
         !tile_offsets_fit(Shape::kRows, Shape::kTokens, w->cols, I8 ? 1 : 2))
       return false;
-    const auto kernel = matmul_tiled_kernel<GATE, RT, CT, W, SLOTS, S, I8, NORM>;
+    const auto kernel = matmul_tiled_kernel<GATE, RT, CT, W, SLOTS, S, I8, NORM, SHORT>;
     if (lds > 64 * 1024) {  // above the default dynamic-LDS cap
       static const hipError_t attr =
           hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -303,15 +303,18 @@ struct TiledLaunch {
     *rc = IE_HIP_OK;
     return true;
   }
-  template <bool GATE, int NR, int CT, int W, int SLOTS, int S>
+  template <bool GATE, int NR, int CT, int W, int SLOTS, int S, bool SHORT = false>
   bool with_types(int* rc) const {
     if constexpr (SLOTS == 8) {  // the folded rmsnorm: matrices below 16 row tiles per unit
       if (norm.weight)
-        return w->int8 ? go<GATE, NR, CT, W, SLOTS, S, true, true>(rc)
-                       : go<GATE, NR, CT, W, SLOTS, S, false, true>(rc);
+        return w->int8 ? go<GATE, NR, CT, W, SLOTS, S, true, true, SHORT>(rc)
+                       : go<GATE, NR, CT, W, SLOTS, S, false, true, SHORT>(rc);
     }
-    return w->int8 ? go<GATE, NR, CT, W, SLOTS, S, true, false>(rc)
-                   : go<GATE, NR, CT, W, SLOTS, S, false, false>(rc);
+    return w->int8 ? go<GATE, NR, CT, W, SLOTS, S, true, false, SHORT>(rc)
+                   : go<GATE, NR, CT, W, SLOTS, S, false, false, SHORT>(rc);
+  }
+  bool run_short(bool gate, int* rc) const {
+    return gate ? with_types<true, 4, 2, 8, 8, 1, true>(rc) : with_types<false, 2, 2, 8, 8, 1, true>(rc);
   }
   template <bool GATE>
   bool run(int shape, int* rc) const {
@@ -401,11 +404,14 @@ int launch_matmul(bool gate, float* y, const float* x, const ie_matrix& w, const
   const int TT = !wide ? 1 : tok_tiles > 2 ? 4 : tok_tiles;
   if ((T + 16 * TT - 1) / (16 * TT) > 65535)
     return fail(IE_HIP_EINVAL, std::string(who) + ": too many tokens");
-  // LDS tiles: K in whole 32-wide blocks, at least one per slot, and 16-byte aligned weights
-  // for the DMA (x always is).
+  // LDS tiles: K in whole 32-wide blocks, at least one per slot or a launch of many tiles, and
+  // 16-byte aligned weights for the DMA (x always is).
   const uintptr_t weights = reinterpret_cast<uintptr_t>(w.data) |
                             reinterpret_cast<uintptr_t>(w2 ? w2->data : nullptr);
-  if (w.cols % 32 == 0 && w.cols >= 32 * waves && ((reinterpret_cast<uintptr_t>(x) | weights) & 15) == 0) {
+  const int64_t tiles = int64_t((w.rows + 15) / 16) * tok_tiles;
+  const bool short_k = w.cols < 32 * waves;
+  const bool staged = !short_k || (!wide && short_k_staged(tiles, w.cols, norm.weight != nullptr, cus));
+  if (w.cols % 32 == 0 && staged && ((reinterpret_cast<uintptr_t>(x) | weights) & 15) == 0) {
     const uintptr_t out = reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(split.y1) |
                           reinterpret_cast<uintptr_t>(split.y2) | reinterpret_cast<uintptr_t>(bias) |
                           reinterpret_cast<uintptr_t>(w.scale) |
@@ -416,6 +422,8 @@ int launch_matmul(bool gate, float* y, const float* x, const ie_matrix& w, const
     bool launched;
     if (wide) {
       launched = launch.run_wide(gate, &rc);
+    } else if (short_k) {
+      launched = launch.run_short(gate, &rc);
     } else {
       const int shape = choose_tile(gate, w.rows, w.cols, T, cus);
       launched = gate ? launch.run<true>(shape, &rc) : launch.run<false>(shape, &rc);
@@ -427,7 +435,6 @@ int launch_matmul(bool gate, float* y, const float* x, const ie_matrix& w, const
   }
   // Direct loads. Tiles per workgroup from the count of 16 x 16 output tiles: two row tiles
   // from 4 per compute unit on, 4 x 4 (or the token tiles there are) for wide matrices.
-  const int64_t tiles = int64_t((w.rows + 15) / 16) * tok_tiles;
   int RT = wide ? 4 : tiles >= 4 * int64_t(cus) ? 2 : 1;
   if (gate) RT = std::min(RT, 2);
   const dim3 grid((w.rows + 16 * RT - 1) / (16 * RT), (T + 16 * TT - 1) / (16 * TT));

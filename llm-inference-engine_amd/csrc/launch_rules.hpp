@@ -91,6 +91,15 @@ inline int choose_tile(bool gate, int rows, int cols, int T, int cus) {
   return best;
 }
 
+// K below a 32-wide block for each of the 8 slots: 32 rows x 32 tokens in LDS from 2 16 x 16 tiles
+// per compute unit on, direct loads below, where a launch's fixed time is all there is (us,
+// one staged 16 x 16 tile / direct / 32 x 32: 256 x 192 at 600 tokens 3.67 / 4.20 / 3.56, 896 x
+// 192 at 4,000 35 / 26 / 17, 4,864 x 96 at 600 25 / 15 / 12; 896 x 192 with the norm at 64
+// 3.9 / 3.9 / 4.8, 896 x 32 with the norm at 600 11.5 / 6.1 / 7.1).
+inline bool short_k_staged(int64_t tiles, int cols, bool norm, int cus) {
+  return tiles >= 2 * int64_t(cus) && (!norm || cols >= 96);
+}
+
 // Whether a tile's byte offsets from its first row and token fit the 32 bits that its loads
 // take them in (128 bf16 rows: up to 16.7 M columns).
 inline bool tile_offsets_fit(int tile_rows, int tile_tokens, int64_t cols, int weight_bytes) {

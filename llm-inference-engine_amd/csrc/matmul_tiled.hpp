@@ -189,7 +189,9 @@ __device__ __forceinline__ void put_rows(const f32x4 (&v)[GATE ? 2 : 1], float i
 // activations, 5.5 instructions a value, done again by every row tile: hence tiles of up to
 // 128 rows; gate/up at 4,000 tokens: VALU issue 61%, matrix cores 36% of the cycles). At few
 // tokens a launch's fixed time and the 16-token tile's split.
-template <bool GATE, int RT, int CT, int W, int SLOTS, int S, bool I8, bool NORM>
+//
+// SHORT: K has fewer blocks than slots; a slot without one adds zeros.
+template <bool GATE, int RT, int CT, int W, int SLOTS, int S, bool I8, bool NORM, bool SHORT>
 __global__ void __launch_bounds__(64 * W)
 matmul_tiled_kernel(float* __restrict__ y, const float* __restrict__ x, const void* __restrict__ w,
                     const float* __restrict__ scale, const void* __restrict__ w2,
@@ -240,7 +242,7 @@ matmul_tiled_kernel(float* __restrict__ y, const float* __restrict__ x, const vo
   const char* const w2base = GATE ? static_cast<const char*>(w2) + size_t(row0) * cols * kWBytes : wbase;
   const char* const xbase = reinterpret_cast<const char*>(x + size_t(tok0) * cols);
 
-  const int nblocks = cols >> 5;  // at least SLOTS (the launcher): every slot has a block
+  const int nblocks = cols >> 5;  // at least SLOTS, unless SHORT (the launcher)
   auto blocks_of = [&](int slot) { return (nblocks - slot + SLOTS - 1) / SLOTS; };
   const int first = blocks_of(wave);  // blocks of this wave's first slot
   const int nsteps = N == 1 ? first : first + blocks_of(wave + W);
@@ -302,6 +304,7 @@ matmul_tiled_kernel(float* __restrict__ y, const float* __restrict__ x, const vo
       for (int i = 0; i < NR; ++i) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     const int end = n == 0 ? first : nsteps;
+    if (SHORT && step == end) continue;
     do {
       wait_steps<S - 1, kPerStep>(nsteps - 1 - step);  // this step's tiles have landed
       const unsigned char* st = stages + stage * Shape::kStage;

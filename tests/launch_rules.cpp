@@ -12,6 +12,9 @@ extern "C" int prefill_f32_kernel(int T, int n_heads, int cus) {
 extern "C" int tile(int gate, int rows, int cols, int T, int cus) {
   return choose_tile(gate != 0, rows, cols, T, cus);
 }
+extern "C" int short_k(int64_t tiles, int cols, int norm, int cus) {
+  return short_k_staged(tiles, cols, norm != 0, cus);
+}
 extern "C" int offsets_fit(int rows, int tokens, int64_t cols, int weight_bytes) {
   return tile_offsets_fit(rows, tokens, cols, weight_bytes);
 }

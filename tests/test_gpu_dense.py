@@ -296,7 +296,7 @@ TILED = [(1, 898, 288), (17, 898, 288), (77, 898, 288), (200, 898, 288), (333, 8
          (600, 898, 288), (1003, 898, 288), (450, 1152, 896), (50, 900, 256), (50, 900, 224),
          (9, 70001, 128), (21, 70001, 160), (16, 70001, 992), (17, 65537, 1024), (33, 70001, 224),
          (64, 65540, 1024), (40, 66000, 1056), (65, 66000, 896), (450, 898, 288), (9, 70001, 928),
-         (33, 70001, 800)]
+         (33, 70001, 800), (333, 898, 32), (333, 898, 96), (1003, 898, 224)]
 
 
 @pytest.mark.parametrize("T,rows,cols", TILED)
@@ -345,7 +345,7 @@ def test_gate_tile_shapes(ie, dev, T, int8):
 # T, rows, cols: every gate/up tile shape with ragged rows (48 rows of two INT8 matrices straddle
 # one 1 KB load), and wide matrices.
 GATE_TILED = [(1, 898, 288), (77, 898, 288), (150, 898, 288), (333, 898, 288), (450, 898, 896),
-              (5, 65530, 160), (37, 65537, 96)]
+              (5, 65530, 160), (37, 65537, 96), (333, 898, 64), (333, 898, 96), (1003, 898, 224)]
 
 
 @pytest.mark.parametrize("T,rows,cols", GATE_TILED)

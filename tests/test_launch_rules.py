@@ -99,3 +99,14 @@ def test_tile_offsets(rules, rows, tokens, cols, wbytes, fits):
     launch goes to the kernel with 64-bit addresses."""
     assert rules.offsets_fit(rows, tokens, ctypes.c_int64(cols), wbytes) == fits
     assert fits == (rows * cols * wbytes < 2**32 and tokens * cols * 4 < 2**32)
+
+
+def test_short_k(rules):
+    """Matrices of fewer than 8 K blocks; the dense tests' shapes take both sides of the line."""
+    staged = lambda T, rows, cols, norm=0: rules.short_k(
+        ctypes.c_int64((rows + 15) // 16 * ((T + 15) // 16)), cols, norm, CUS)
+    assert staged(600, 256, 192) and staged(4000, 64, 32) and staged(600, 896, 96, 1)
+    assert not (staged(64, 896, 192) or staged(600, 64, 192) or staged(600, 896, 64, 1))
+    short = [s for s in dense.TILED if s[2] < 256 and s[1] < 65000]
+    assert {staged(*s) for s in short} == {0, 1}
+    assert any(staged(*s) and s[2] % 256 for s in short) and any(staged(*s) for s in dense.GATE_TILED)
