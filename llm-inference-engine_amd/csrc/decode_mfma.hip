@@ -68,6 +68,7 @@
 
 #include "common.hpp"
 #include "decode.hpp"
+#include "launch_rules.hpp"
 #include "mfma.hpp"
 
 namespace iehip {
@@ -606,9 +607,9 @@ decode_partial_mfma(float* __restrict__ out, float* __restrict__ part_o,
 // One workgroup per (row, chunk), the grid numbered as for the 16-bit kernel; its W waves
 // take the chunk's pages in turn and merge their (o, m, l) through LDS. A page is a chain of
 // 64 matrix instructions of 32 cycles and the round trip of its 16 KB, ~1 us for a wave by
-// itself, so most chunk sizes take 4 waves (48 rows of 256 to 2,048 positions in chunks of
+// itself, so most chunk sizes take 2 or 4 waves (48 rows of 256 to 2,048 positions in chunks of
 // 128 were 455 waves on 1,024 SIMDs: 19.5 -> 12.0 us under the profiler's trace, 21.9 -> 18.4
-// with the merge); see decode_mfma_f32 for the sizes that take one. The count follows from
+// with the merge); see decode_f32_waves. The count follows from
 // the chunk size alone, so a row's result does not depend on the launch.
 constexpr int kPageF32 = 16 * kKvd * 4;  // bytes of one f32 page of one pool
 
@@ -954,16 +955,11 @@ int decode_mfma_f32(float* out, const float* q, const void* k_pool, const void* 
                        row_seq, kv.tables, T, kv.max_pages, kv.num_pages, n_heads,
                        n_heads / n_kv_heads, num_chunks, chunk_tokens, plan);
   };
-  // Waves per chunk, from its size alone (us; rows x positions, f32): 192 positions are
-  // chosen where workgroups abound (64 x 128-4,096: one wave 28.8, four 32.0), 32 hold two
-  // pages (16 x 512-2,048: 11.5 against 15.7); 64 and 128 are chosen for small grids
-  // (16 x 512-2,048 at 64: 12.4 against 12.0; 48 x 256-2,048 at 128: 19.6 against 18.4), and a
-  // chunk of more than 192 is a long chain for one wave (16 x 512-2,048 at 256: 26.6 against
-  // 15.7).
-  if (chunk_tokens <= 32 || (chunk_tokens > 128 && chunk_tokens <= 192))
-    launch(decode_partial_mfma_f32<1>, 1);
-  else
-    launch(decode_partial_mfma_f32<4>, 4);
+  switch (decode_f32_waves(chunk_tokens)) {
+    case 1: launch(decode_partial_mfma_f32<1>, 1); break;
+    case 2: launch(decode_partial_mfma_f32<2>, 2); break;
+    default: launch(decode_partial_mfma_f32<4>, 4);
+  }
   if (int rc = check_launch("attention_mfma_f32")) return rc;
   return decode_merge(out, ws, row_pos, T, n_heads, num_chunks, chunk_tokens, stream);
 }

@@ -125,4 +125,17 @@ inline WideKernel choose_wide(bool gate, int cols, int T) {
                                                           : WideKernel::kTiles32;
 }
 
+// Waves per chunk of an f32 cache's decode, from the chunk's size alone, so that a row's result
+// does not depend on the launch. attention_chunk_tokens chooses 192 where workgroups abound and
+// 32, 64 and 128 for small grids (us; rows x positions): 192: 64 x 128-4,096 one wave 28.8, four
+// 32.0; 32, two pages: 16 x 512-2,048 11.5, four 15.7; 64: 16 x 512-2,048 four 12.2, two 12.9, one
+// 12.7; 128: 48 x 256-2,048 four 18.4, one 19.6. Between those, two waves waste least where the grid
+// is large and lose little where it is not (48: 1,024 x 16-512 one 61, two 64, four 85, 1 x 600 9.8,
+// 9.4 and 8.9; 96: 256 x 1,024-4,096 139, 138 and 148). More than 192 is a long chain for one
+// wave (256: 16 x 512-2,048 26.6, four 15.7).
+inline int decode_f32_waves(int chunk_tokens) {
+  if (chunk_tokens <= 32 || (chunk_tokens > 128 && chunk_tokens <= 192)) return 1;
+  return chunk_tokens != 64 && chunk_tokens <= 96 ? 2 : 4;
+}
+
 }  // namespace iehip

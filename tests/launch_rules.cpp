@@ -15,6 +15,7 @@ extern "C" int tile(int gate, int rows, int cols, int T, int cus) {
 extern "C" int short_k(int64_t tiles, int cols, int norm, int cus) {
   return short_k_staged(tiles, cols, norm != 0, cus);
 }
+extern "C" int decode_waves(int chunk_tokens) { return decode_f32_waves(chunk_tokens); }
 extern "C" int offsets_fit(int rows, int tokens, int64_t cols, int weight_bytes) {
   return tile_offsets_fit(rows, tokens, cols, weight_bytes);
 }

@@ -434,7 +434,7 @@ def test_batch_shapes(ie, O, dev, case, kv):
         assert np.all(got[~live] == 7.0), "rows with position -1 must be left untouched"
 
 
-@pytest.mark.parametrize("chunk_tokens", [16, 32, 48, 64, 128, 144, 192, 208, 1024])
+@pytest.mark.parametrize("chunk_tokens", [16, 32, 48, 64, 80, 128, 144, 192, 208, 1024])
 @pytest.mark.parametrize("planned", [False, True])
 def test_f32_waves_per_chunk(ie, O, dev, chunk_tokens, planned):
     """f32 caches: every wave count per chunk, with chunks whose pages do not divide among the

@@ -110,3 +110,9 @@ def test_short_k(rules):
     short = [s for s in dense.TILED if s[2] < 256 and s[1] < 65000]
     assert {staged(*s) for s in short} == {0, 1}
     assert any(staged(*s) and s[2] % 256 for s in short) and any(staged(*s) for s in dense.GATE_TILED)
+
+
+def test_decode_f32_waves(rules):
+    got = {c: rules.decode_waves(c) for c in (16, 32, 48, 64, 80, 96, 112, 128, 144, 192, 208, 1024)}
+    assert got == {16: 1, 32: 1, 48: 2, 64: 4, 80: 2, 96: 2, 112: 4, 128: 4, 144: 1, 192: 1, 208: 4,
+                   1024: 4}
