@@ -152,7 +152,7 @@ def _native():
         spec = importlib.util.spec_from_file_location("native_calls", CALLS_PATH)
         calls = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(calls)
-        calls.set_dtypes(torch.float32, torch.float16, torch.bfloat16)
+        calls.set_types(torch.float32, torch.float16, torch.bfloat16, Matrix)
         _calls = calls
     return _calls
 

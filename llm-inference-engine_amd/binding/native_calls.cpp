@@ -4,10 +4,10 @@
 // same call here 1.9 us (matmul 1.9 and 0.8): with the launches' own 5 us, the difference
 // between a host-bound and a GPU-bound decode step of one sequence (8-10 us).
 //
-// Arguments are the C function's, in order: a pointer is None, an address or an object with
-// data_ptr() (a tensor); an ie_kv_layout is (tables, max_pages, pool, elements per token row);
-// an ie_matrix any 32-byte buffer (the ctypes Matrix). The status code is returned. The GIL is
-// released during the call, as ctypes does.
+// Arguments are the C function's, in order: a pointer is None or an object with data_ptr() (a
+// tensor), a stream None or its handle, an integer a Python int; an ie_kv_layout is (tables,
+// max_pages, pool, elements per token row); an ie_matrix the ctypes Matrix. The status code is
+// returned. The GIL is released during the call, as ctypes does.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -20,42 +20,65 @@
 
 namespace {
 
-// The torch dtypes of IE_KV_F32, IE_KV_F16, IE_KV_BF16 (set_dtypes).
+// The torch dtypes of IE_KV_F32, IE_KV_F16, IE_KV_BF16, and the Matrix class (set_types).
 PyObject* g_dtypes[3] = {nullptr, nullptr, nullptr};
+PyObject* g_matrix = nullptr;
 PyObject *g_data_ptr = nullptr, *g_numel = nullptr, *g_dtype = nullptr;
 
 bool as_u64(PyObject* o, unsigned long long* v) {
-  if (PyLong_Check(o)) {
-    *v = PyLong_AsUnsignedLongLongMask(o);
-  } else {
-    PyObject* i = PyNumber_Index(o);
-    if (!i) return false;
-    *v = PyLong_AsUnsignedLongLongMask(i);
-    Py_DECREF(i);
+  if (!PyLong_Check(o)) {
+    PyErr_Format(PyExc_TypeError, "int expected instead of %s instance", Py_TYPE(o)->tp_name);
+    return false;
   }
+  *v = PyLong_AsUnsignedLongLongMask(o);
   return !(*v == ~0ull && PyErr_Occurred());
+}
+
+// elements // (IE_HIP_PAGE_SIZE * row), as Python divides: any row, rounded down.
+bool pages_of(unsigned long long elements, PyObject* row, int32_t* pages) {
+  if (!PyLong_Check(row)) {
+    PyErr_Format(PyExc_TypeError, "int expected instead of %s instance", Py_TYPE(row)->tp_name);
+    return false;
+  }
+  int over = 0;
+  const long long r = PyLong_AsLongLongAndOverflow(row, &over), e = static_cast<long long>(elements);
+  constexpr long long kMost = (1ll << 62) / IE_HIP_PAGE_SIZE;
+  if (!over && r == 0) {
+    PyErr_SetString(PyExc_ZeroDivisionError, "a token row has no elements");
+    return false;
+  }
+  if (over > 0 || r > kMost) {
+    *pages = 0;
+  } else if (over < 0 || r < -kMost) {
+    *pages = e ? -1 : 0;
+  } else {
+    const long long d = r * IE_HIP_PAGE_SIZE;
+    *pages = int32_t(e / d - (d < 0 && e % d != 0));
+  }
+  return true;
 }
 
 bool address(PyObject* o, void** p) {
   *p = nullptr;
   if (o == Py_None) return true;
   unsigned long long v = 0;
-  if (PyLong_Check(o)) {
-    if (!as_u64(o, &v)) return false;
-  } else {
-    PyObject* r = PyObject_CallMethodNoArgs(o, g_data_ptr);
-    if (!r) return false;
-    const bool ok = as_u64(r, &v);
-    Py_DECREF(r);
-    if (!ok) return false;
-  }
+  PyObject* r = PyObject_CallMethodNoArgs(o, g_data_ptr);
+  if (!r) return false;
+  const bool ok = as_u64(r, &v);
+  Py_DECREF(r);
+  if (!ok) return false;
   *p = reinterpret_cast<void*>(static_cast<uintptr_t>(v));
   return true;
 }
 
 template <class T>
 bool convert(PyObject* o, T* out) {
-  if constexpr (std::is_pointer_v<T>) {
+  if constexpr (std::is_same_v<T, hipStream_t>) {
+    unsigned long long v = 0;
+    if (o != Py_None && !as_u64(o, &v)) return false;
+    *out = reinterpret_cast<T>(static_cast<uintptr_t>(v));
+    return true;
+  } else if constexpr (std::is_pointer_v<T>) {
     void* p;
     if (!address(o, &p)) return false;
     *out = reinterpret_cast<T>(p);
@@ -71,6 +94,11 @@ bool convert(PyObject* o, T* out) {
     *out = static_cast<T>(v);
     return true;
   } else if constexpr (std::is_same_v<T, ie_matrix>) {
+    const int is = PyObject_IsInstance(o, g_matrix);
+    if (is <= 0) {
+      if (!is) PyErr_SetString(PyExc_TypeError, "expected a Matrix");
+      return false;
+    }
     Py_buffer b;
     if (PyObject_GetBuffer(o, &b, PyBUF_SIMPLE)) return false;
     const bool ok = b.len == Py_ssize_t(sizeof(ie_matrix));
@@ -85,10 +113,9 @@ bool convert(PyObject* o, T* out) {
       return false;
     }
     void* tables;
-    unsigned long long max_pages, row, elements;
+    unsigned long long max_pages, elements;
     PyObject* pool = PyTuple_GET_ITEM(o, 2);
-    if (!address(PyTuple_GET_ITEM(o, 0), &tables) || !as_u64(PyTuple_GET_ITEM(o, 1), &max_pages) ||
-        !as_u64(PyTuple_GET_ITEM(o, 3), &row))
+    if (!address(PyTuple_GET_ITEM(o, 0), &tables) || !as_u64(PyTuple_GET_ITEM(o, 1), &max_pages))
       return false;
     PyObject* n = PyObject_CallMethodNoArgs(pool, g_numel);
     if (!n) return false;
@@ -101,13 +128,10 @@ bool convert(PyObject* o, T* out) {
       if (dtype == g_dtypes[i]) code = i;
     if (code < 0) PyErr_SetObject(PyExc_KeyError, dtype);
     Py_DECREF(dtype);
-    if (code < 0) return false;
-    if (row == 0) {
-      PyErr_SetString(PyExc_ZeroDivisionError, "a token row has no elements");
-      return false;
-    }
+    int32_t pages;
+    if (code < 0 || !pages_of(elements, PyTuple_GET_ITEM(o, 3), &pages)) return false;
     *out = ie_kv_layout{static_cast<const int32_t*>(tables), int32_t(max_pages), IE_HIP_PAGE_SIZE,
-                        int32_t(code), int32_t(elements / (IE_HIP_PAGE_SIZE * row))};
+                        int32_t(code), pages};
     return true;
   }
 }
@@ -120,9 +144,16 @@ struct Args<R (*)(A...)> {
   static constexpr size_t count = sizeof...(A);
 };
 
+template <bool kMatrices, class T>
+bool convert_if(PyObject* o, T* out) {
+  return std::is_same_v<T, ie_matrix> != kMatrices || convert(o, out);
+}
+
+// Matrices first: their check asks no tensor for anything.
 template <class T, size_t... I>
 bool convert_all(PyObject* const* args, T& t, std::index_sequence<I...>) {
-  return (convert(args[I], &std::get<I>(t)) && ...);
+  return (convert_if<true>(args[I], &std::get<I>(t)) && ...) &&
+         (convert_if<false>(args[I], &std::get<I>(t)) && ...);
 }
 
 template <auto Fn>
@@ -141,11 +172,13 @@ PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return PyLong_FromLong(rc);
 }
 
-PyObject* set_dtypes(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  if (n != 3) {
-    PyErr_SetString(PyExc_TypeError, "expected the dtypes of f32, f16 and bf16");
+PyObject* set_types(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  if (n != 4) {
+    PyErr_SetString(PyExc_TypeError, "expected the dtypes of f32, f16 and bf16 and the Matrix class");
     return nullptr;
   }
+  Py_INCREF(args[3]);
+  Py_XSETREF(g_matrix, args[3]);
   for (int i = 0; i < 3; ++i) {
     Py_INCREF(args[i]);
     Py_XSETREF(g_dtypes[i], args[i]);
@@ -156,7 +189,7 @@ PyObject* set_dtypes(PyObject*, PyObject* const* args, Py_ssize_t n) {
 #define IE_CALL(name) \
   {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(&call<&name>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    {"set_dtypes", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(&set_dtypes)), METH_FASTCALL,
+    {"set_types", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(&set_types)), METH_FASTCALL,
      nullptr},
     IE_CALL(ie_hip_rope_and_cache),
     IE_CALL(ie_hip_attention),

@@ -160,3 +160,38 @@ def test_native_calls(ie):
         calls.ie_hip_matmul(0, 0)
     with pytest.raises(TypeError):
         calls.ie_hip_matmul(0, 0, b"short", None, 0, 0, 0)
+
+
+def test_native_calls_refuse_what_ctypes_refused(ie):
+    """Numbers for tensors, other buffers for a Matrix, floats and numpy integers for ints; and
+    head counts whose product passes 64 bits, which the pages are still divided by as Python
+    divides (none left: refused by the library, not a division fault)."""
+    import numpy as np
+    import torch
+    z = torch.zeros
+    stream = type("S", (), {"cuda_stream": 0})()
+    w = ie.matrix(z(16, 32, dtype=torch.bfloat16))
+    calls = ie._native()
+    for y in (5, 0, 5.0, "y", b"y"):
+        with pytest.raises(AttributeError):
+            ie.rmsnorm(y, z(1, 32), z(32), 1e-6, stream=stream)
+        with pytest.raises(AttributeError):
+            ie.matmul(z(1, 16), z(1, 32), w, bias=y, stream=stream)
+    for other in (bytes(32), bytearray(32), np.zeros(4), memoryview(bytes(w)), None, 0):
+        with pytest.raises(TypeError):
+            calls.ie_hip_matmul(z(1, 16), z(1, 32), other, None, 0, 0, 0)
+    for dim in (32.0, np.int64(32), None):
+        with pytest.raises(TypeError):
+            calls.ie_hip_rmsnorm(z(0, 32), z(0, 32), z(32), 0, dim, 1e-6, 0)
+    one, kp = z(1, dtype=torch.int32), z(64, 128, dtype=torch.float16)
+
+    def append(n_kv, head_dim=64):
+        ie.rope_and_cache(None, z(1, 128), z(1, 128), kp, kp, z(4, 64), one, one, one, 1, 14, n_kv,
+                          head_dim, stream=stream)
+    for n_kv in (2**54, 2**58, 2**60, 2**70, -2, -2**58, -2**70, 1000):  # no page, or less than one
+        with pytest.raises(ie.IeHipError):
+            append(n_kv)
+    with pytest.raises(ZeroDivisionError):
+        append(0)
+    with pytest.raises(TypeError):
+        append(2.0)
