@@ -778,9 +778,9 @@ def bench_mixed(args, torch, ie, O):
                else ms_pfp)
     ms_dec2 = time_steps(torch, decode_two_calls, args.steps, args.warmup, stream) if fused else ms_dec
     flops = 4 * NH * HD * P * (P + 1) // 2
-    # Dense matrix peak of the type the prefill tiles run in: the 16-bit MFMA for
-    # f16/bf16 caches, the fp32 MFMA for f32 caches (MI355X published figures).
-    mfma_peak = 157.3 if kv == "f32" else 2500.0
+    # Dense matrix peak of what the prefill tiles run on: the 16-bit MFMA (MI355X published
+    # figure); for f32 caches six bf16 products make a float32 one.
+    mfma_peak = round(2500.0 / 6, 1) if kv == "f32" else 2500.0
     tflops = flops / (ms_pf * 1e-3) / 1e12
     dec_bytes = decode_bytes([lens[s] + 1 for s in dec], KV_BYTES[kv])
     res = {

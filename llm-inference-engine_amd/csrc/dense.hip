@@ -19,7 +19,8 @@
 // matmul_tiled_kernel (matmul_tiled.hpp) is that product with its operands staged in LDS,
 // in one of several tile shapes (see choose_tile), for K in whole 32-wide blocks and
 // weights aligned for the DMA; matmul_mfma_kernel here loads its operands directly, for
-// every other shape. Both add every output in the same order, fixed by the matrix alone.
+// every other shape (launch_rules.hpp says which). Both add every output in the same order,
+// fixed by the matrix alone.
 // Lane (g, r) of a tile: A = W[row r][k + 8g .. +8], B = x[token r][k + 8g ..
 // +8]; the result lane holds rows 4g .. 4g+3 of token r.
 #include <algorithm>

@@ -20,13 +20,13 @@ enum class PrefillKernel { kPairsTwoTeams, kPairsOneTeam, kRows1x8, kRows2x8, kR
 // head). Measured (us, f16 / bf16; rows on cached positions), pairs of blocks against row
 // blocks: 4,000 on 0: 54 / 82 against 68 / 95; 2,000 on 0: 31 / 46 against 28 / 34; 2,000 on
 // 2,000: 67 / 107 against 54 / 73; 600 on 0: 18 / 23 against 11 / 12; 130 on 4,000: 81 / 135
-// against 17 / 19; 2,720 on 0: 36.7 / 62 against 37.7 / 52; 64/8 heads, 512 on 0: 17.8 / 23
-// against 17.3 / 20, 640 on 0: 18.6 / 23.7 against 23.8 / 27.1.
+// against 17 / 19; 2,720 on 0: 37.0 / 55.7 against 37.7 / 47.4; 64/8 heads, 512 on 0: 17.4 / 21.7
+// against 17.2 / 19.2, 640 on 0: 18.7 / 23.8 against 23.9 / 27.3.
 // Of the row-block shapes: one block and 8 waves while that gives at most a workgroup per unit
 // (64 on 2,000, f16: 11.1, two blocks 13); two blocks, 32-key tiles and 8 waves up to 2.5 (512
 // on 8,000, f16: 37, 4 waves 53), or up to the 2 that a unit holds at once where the few that
-// come after those hold the launch up (hi + lo operands: 1,280 on 0 22.0, 4 waves 17.2; on
-// 4,000 78 and 76; short prompts of small groups: 32/8 heads, f16, 576 on 0 16.6, 4 waves
+// come after those hold the launch up (hi + lo operands, 1,280 on 0: 22.0, 4 waves 17.2; on
+// 4,000 79.5 and 77.7; short prompts of small groups: 32/8 heads, f16, 576 on 0 16.6, 4 waves
 // 14.0); 64-key tiles and 4 waves above (2,000 on 2,000, bf16: 73, 8 waves 77).
 // Two teams of waves split a pair's key tiles while the pairs leave units without a workgroup
 // or with one: twice the waves, half the chain of tiles of each.

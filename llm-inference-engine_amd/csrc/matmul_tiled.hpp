@@ -196,7 +196,8 @@ __device__ __forceinline__ void put_rows(const f32x4 (&v)[GATE ? 2 : 1], float i
 //
 // What bounds it: at many tokens the VALU and matrix cores in turn (the x3 split of the
 // activations, 5.5 instructions a value, done again by every row tile: hence tiles of up to
-// 128 rows; gate/up at 4,000 tokens: VALU issue 61%, matrix cores 36% of the cycles). At few
+// 128 rows; norm + gate/up at 4,000 tokens: VALU issue 54%, matrix cores 36% of the cycles, and
+// with INT8 weights, widened again by every token tile, 60 and 30%). At few
 // tokens a launch's fixed time and the 16-token tile's split.
 //
 // SHORT: K has fewer blocks than slots; a slot without one adds zeros.

@@ -1112,20 +1112,21 @@ prefill_rows_kernel(float* __restrict__ out, const float* __restrict__ q,
 
 // ---------------------------------------------------------------------------
 // float32 KV caches. Queries, keys, weights and values enter the 16-bit matrix cores in
-// three bf16 parts each, x = hi + mid + lo exactly (split3), and every product is the six
-// largest of the nine partial ones: what is left out is below 2^-26 of the product, under
-// the rounding of its float32 sum. (Measured against float64: 4.4e-7 at 1,333 rows on 1,000
-// cached, where v_mfma_f32_16x16x4_f32 on the whole float32 values gave 8.0e-7.) The f32
-// instruction takes 256 cycles for the 16x16x32 product that six bf16 ones do in 96, and no
-// VALU instruction runs beside it (probe: 52 cycles with four VALU instructions beside it,
-// 35 alone), while the bf16 ones leave the VALU free for the splits and the softmax.
+// three bf16 parts each, x = hi + mid + lo exactly (split3; for what has no such split see
+// `redo` at the end), and every product is the six largest of the nine partial ones: what is
+// left out is at most about 2^-24 of the product (parts of up to 2^-8 and 2^-17 of a value), a
+// float32 rounding of it. The whole is as exact as float32 products: against float64 4.4e-7 at
+// 1,333 rows on 1,000 cached, where v_mfma_f32_16x16x4_f32 on the whole values gave 8.0e-7.
+// The f32 instruction takes 256 cycles for the 16x16x32 product that six bf16 ones do in 96,
+// and the bf16 ones leave the VALU free for the splits and the softmax.
 //
 // One workgroup per (NB blocks of 16 rows, query head); its waves take 32-key tiles in turn,
 // each with its own K stage, softmax state and output, merged through LDS at the end: no
 // barrier and no sharing until then, and T / 16 / NB x heads workgroups, the longest
 // contexts first, where a workgroup per pair of blocks and KV head left two thirds of the
-// compute units idle at 1,333 rows. What bounds it now is VALU issue: a tile's K and V take
-// 352 instructions to split, shared by NB blocks. Times (us, was 7 waves on shared f32
+// compute units idle at 1,333 rows. What bounds it now: a tile's K and V take 352 VALU
+// instructions to split, shared by NB blocks and done again by every query head; VALU issue
+// takes 50% of the cycles at 1,333 rows on 1,000, the matrix cores 28%, in turn for the most part. Times (us, was 7 waves on shared f32
 // tiles): 1,333 rows on 1,000 cached 237 -> 72, 4,000 rows 281 -> 193, 130 rows on 4,000
 // cached 548 -> 44.
 //   S^T[16 keys x 16 rows] per key group of 16: step ks takes dims 16g + 8ks .. +7, so lane
@@ -1137,8 +1138,9 @@ prefill_rows_kernel(float* __restrict__ out, const float* __restrict__ q,
 //     scores and used after the softmax. Lane (g, r) ends up with row r's dims
 //     16g + 4t + mt (o[mt][t]).
 // K tiles (8 KB) come through LDS by DMA, one stage per wave: read whole into registers,
-// then the next tile is sent for. Loads take a scalar page base and a 32-bit lane offset
-// (64-bit lane addresses: 1,000 rows 30.6 -> 29.5 us, 4,000 rows 198 -> 193). Four waves a
+// then the next tile is sent for. K loads take a scalar page base and a 32-bit lane offset, V
+// loads a 64-bit lane address made from the two (both from 64-bit lane pointers: 1,000 rows
+// 30.6 -> 29.5 us, 4,000 rows 198 -> 193). Four waves a
 // SIMD with one block need its registers at 128, as asked for; three with two blocks spill
 // (1,000 rows 30.6, 4,000 rows 189: not kept); three or four blocks hold so many registers
 // that too few waves are left (4,000 rows 242 and 236 us). K rows are stored with their 16-byte pieces swizzled

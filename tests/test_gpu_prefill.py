@@ -3,8 +3,7 @@
 Same tolerances as decode (f32: rel 1e-5; f16/bf16: 2e-3 abs). Cases: the
 reference self-test's prompts (src/cuda/cuda_runner.cu:920-934: 1, 17, 300,
 1000 rows; a prompt continuing at 500; the 2nd of 2 sequences), a prompt whose
-keys run past 32,768 (the kernels stage page ids 512 tiles at a time), and the
-4,000-token prefill of BASELINE config 5, appended into fresh pages of a
+keys run past 32,768, and the 4,000-token prefill of BASELINE config 5, appended into fresh pages of a
 churned pool with the fused RoPE+append kernel first (all 4,000 rows checked
 against the oracle). Decode and prefill kernels must agree on the same rows. The
 f16 prefill's single rounding of P is checked at its worst: rows with few keys
@@ -48,7 +47,7 @@ PROMPTS = [
     ([540], 0, 500, 40),          # a prompt continuing at 500
     ([100, 300], 1, 0, 300),     # the 2nd of 2 sequences
     ([129], 0, 63, 66),          # starts mid-tile, crosses tile edges
-    ([32830], 0, 32750, 80),     # keys past 32,768: the page ids are staged in two segments
+    ([32830], 0, 32750, 80),     # keys past 32,768
 ]
 
 
@@ -79,8 +78,8 @@ SPLITS = [(0, 2), (500, 33), (77, 335), (3, 1030), (130, 1500)]
 @pytest.mark.parametrize("start,T", SPLITS)
 @pytest.mark.parametrize("hole", [False, True])
 def test_work_splits(ie, O, dev, kv, start, T, hole):
-    """Every split of the prefill's rows and key tiles over workgroups and waves, with NaN in
-    every cached row that no position holds; `hole` puts one page of the sequence outside
+    """Every split of the row-block kernels' rows and key tiles over workgroups and waves (the
+    pair kernel's: test_gpu_prefill_forms.py), with NaN in every cached row that no position holds; `hole` puts one page of the sequence outside
     the pool (its keys are skipped), checked against the sequence with those keys moved out
     of sight."""
     kvt = KVS[kv]
@@ -306,8 +305,8 @@ def test_config5_mixed_step_into_churned_pool(ie, O, dev, kv, impl):
 @pytest.mark.parametrize("kv", list(KVS))
 def test_mfma_forced(ie, O, dev, kv):
     """IMPL_MFMA runs the matrix-core prefill kernels for every KV type: 16-bit caches
-    in their own type (f16: q and P rounded once; bf16: hi + lo operands), f32 caches on
-    the f32 matrix instructions."""
+    in their own type (f16: q and P rounded once; bf16: hi + lo operands), f32 caches in
+    three bf16 parts."""
     kvt = KVS[kv]
     rng = np.random.default_rng(41)
     tables, max_pages, num_pages = make_tables([333], rng)
