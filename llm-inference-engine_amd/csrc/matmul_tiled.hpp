@@ -7,8 +7,6 @@
 
 namespace iehip {
 
-using bf16 = __bf16;
-
 // Outputs: rows [0, split0) go to y ([T, split0]), rows [split0, split1) to y1
 // ([T, split1 - split0]) and the rest to y2 ([T, rows - split1]); a plain
 // matmul has split0 = split1 = rows.
@@ -28,38 +26,6 @@ struct RowNorm {
   const float* weight;  // [cols]
   float eps;
 };
-
-// 8 activations as three bf16 operands whose sum is exact. Pairs are converted and
-// widened back together: 5.5 VALU instructions per value.
-__device__ __forceinline__ void split3(const float4 p, const float4 q, bf16x8& hi, bf16x8& mid,
-                                       bf16x8& lo) {
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-  auto pack = [](float a, float b) {
-    return __builtin_bit_cast(uint32_t, bf16x2{static_cast<bf16>(a), static_cast<bf16>(b)});
-  };
-  auto rest = [](float v, uint32_t h, bool odd) {
-    return v - __uint_as_float(odd ? h & 0xFFFF0000u : h << 16);
-  };
-  const float v[8] = {p.x, p.y, p.z, p.w, q.x, q.y, q.z, q.w};
-  u32x4 h, m, l;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    // The empty asm keeps each packed pair as it is: otherwise every value is
-    // converted once more by itself to be widened (7.5 instructions per value).
-    uint32_t hb = pack(v[2 * j], v[2 * j + 1]);
-    asm("" : "+v"(hb));
-    const float r0 = rest(v[2 * j], hb, false), r1 = rest(v[2 * j + 1], hb, true);
-    uint32_t mb = pack(r0, r1);
-    asm("" : "+v"(mb));
-    h[j] = hb;
-    m[j] = mb;
-    l[j] = pack(rest(r0, mb, false), rest(r1, mb, true));
-  }
-  hi = __builtin_bit_cast(bf16x8, h);
-  mid = __builtin_bit_cast(bf16x8, m);
-  lo = __builtin_bit_cast(bf16x8, l);
-}
 
 // 8 INT8 weights as bf16 (exact for |q| <= 127).
 __device__ __forceinline__ bf16x8 widen_i8(const uint2 raw) {

@@ -55,7 +55,6 @@
 
 #include "common.hpp"
 #include "launch_rules.hpp"
-#include "matmul_tiled.hpp"
 #include "mfma.hpp"
 #include "prefill.hpp"
 
