@@ -680,7 +680,8 @@ inline int64_t unit_grid(int64_t n_units, int n_heads, int n_kv_heads, int threa
 // lane; o[b][mt][t] is dim 16g + 4t + mt. after(b, w, x, dst) follows dims
 // 16g + 4w .. of block b's result x into `out`.
 // n_tiles == 1: only wave 0 took keys, and writes its own result (32/8 heads, 2 rows: 5.7 us
-// through the merge, 4.7, by pairs 5.3). The f32 kernel, which has no registers to spare for that, gives kTeams.
+// through the merge, 4.7, by pairs 5.3). The f32 kernel has no registers to spare for that and
+// gives kTeams.
 template <int NB, int kTeams, typename After>
 __device__ __forceinline__ void merge_teams(unsigned char* smem, float* out, const f32x4 (&o)[NB][4],
                                             const float (&m)[NB], const float (&l)[NB], int t0,
@@ -1125,9 +1126,9 @@ prefill_rows_kernel(float* __restrict__ out, const float* __restrict__ q,
 // contexts first, where a workgroup per pair of blocks and KV head left two thirds of the
 // compute units idle at 1,333 rows. What bounds it now: a tile's K and V take 352 VALU
 // instructions to split, shared by NB blocks and done again by every query head; VALU issue
-// takes 50% of the cycles at 1,333 rows on 1,000, the matrix cores 28%, in turn for the most part. Times (us, was 7 waves on shared f32
-// tiles): 1,333 rows on 1,000 cached 237 -> 72, 4,000 rows 281 -> 193, 130 rows on 4,000
-// cached 548 -> 44.
+// takes 50% of the cycles at 1,333 rows on 1,000, the matrix cores 28%, in turn for the most
+// part. Times (us, was 7 waves on shared f32 tiles): 1,333 rows on 1,000 cached 237 -> 72,
+// 4,000 rows 281 -> 193, 130 rows on 4,000 cached 548 -> 44.
 //   S^T[16 keys x 16 rows] per key group of 16: step ks takes dims 16g + 8ks .. +7, so lane
 //     (g, r) reads key r's dims 16g .. 16g+15 (64 bytes, 4 LDS reads).
 //   O^T[64 dims x 16 rows] += V^T . P^T: one step of 32 keys; lane (g, r)'s B operand is its
@@ -1139,12 +1140,11 @@ prefill_rows_kernel(float* __restrict__ out, const float* __restrict__ q,
 // K tiles (8 KB) come through LDS by DMA, one stage per wave: read whole into registers,
 // then the next tile is sent for. K loads take a scalar page base and a 32-bit lane offset, V
 // loads a 64-bit lane address made from the two (both from 64-bit lane pointers: 1,000 rows
-// 30.6 -> 29.5 us, 4,000 rows 198 -> 193). Four waves a
-// SIMD with one block need its registers at 128, as asked for; three with two blocks spill
-// (1,000 rows 30.6, 4,000 rows 189: not kept); three or four blocks hold so many registers
-// that too few waves are left (4,000 rows 242 and 236 us). K rows are stored with their 16-byte pieces swizzled
-// (piece ^ (key & 15)), so the 16 lanes of a group reading the same dims of 16 keys hit
-// distinct banks.
+// 30.6 -> 29.5 us, 4,000 rows 198 -> 193). Four waves a SIMD with one block need its registers
+// at 128, as asked for; three with two blocks spill (1,000 rows 30.6, 4,000 rows 189: not
+// kept); three or four blocks hold so many registers that too few waves are left (4,000 rows
+// 242 and 236 us). K rows are stored with their 16-byte pieces swizzled (piece ^ (key & 15)),
+// so the 16 lanes of a group reading the same dims of 16 keys hit distinct banks.
 constexpr int kKeysF32 = 32;                      // keys per wave tile (2 pages)
 constexpr int kStageF32 = kKeysF32 * 64 * 4;      // 8 KB of K
 // The six products of two operands in three parts (0 the largest), the smallest first.

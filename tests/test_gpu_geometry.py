@@ -4,8 +4,9 @@ The kernels are written for the reference's limits (head_dim 64 for attention,
 at most 8 query heads per KV head; head_dim 64 or 128 for RoPE + append), with
 the matrix-core decode kernel taking rows of 128 KV elements and up to 16 query
 heads. These cases run such geometries (the prefill's forms per group size:
-test_gpu_prefill_forms.py) against the oracle at the same tolerances as the Qwen tests (f32: the reference's compare()
-<= 1e-5; f16/bf16: 2e-3 absolute), through both implementations.
+test_gpu_prefill_forms.py) against the oracle at the same tolerances as the Qwen
+tests (f32: the reference's compare() <= 1e-5; f16/bf16: 2e-3 absolute), through both
+implementations.
 """
 from __future__ import annotations
 

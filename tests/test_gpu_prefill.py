@@ -79,9 +79,9 @@ SPLITS = [(0, 2), (500, 33), (77, 335), (3, 1030), (130, 1500)]
 @pytest.mark.parametrize("hole", [False, True])
 def test_work_splits(ie, O, dev, kv, start, T, hole):
     """Every split of the row-block kernels' rows and key tiles over workgroups and waves (the
-    pair kernel's: test_gpu_prefill_forms.py), with NaN in every cached row that no position holds; `hole` puts one page of the sequence outside
-    the pool (its keys are skipped), checked against the sequence with those keys moved out
-    of sight."""
+    pair kernel's: test_gpu_prefill_forms.py), with NaN in every cached row that no position
+    holds; `hole` puts one page of the sequence outside the pool (its keys are skipped),
+    checked against the sequence with those keys moved out of sight."""
     kvt = KVS[kv]
     rng = np.random.default_rng(start + T)
     n = start + T
